@@ -215,6 +215,22 @@ static std::vector<int32_t> cube_embed(int p) {
   return e;
 }
 
+// whether 3 x n points (n boundary points of the m^3 lattice) lie on a centred lattice, to
+// rounding: coordinate i of the lattice at a (2 i / (m - 1) - 1), a that of the last point
+static bool on_lattice(const double *x, int m) {
+  const int n = m * m * m - (m - 2) * (m - 2) * (m - 2);
+  const double a = x[3 * (n - 1)];
+  int q = 0;
+  for (int k = 0; k < m * m * m; k++) {
+    const int i[3] = {k % m, (k / m) % m, k / (m * m)};
+    if (!(i[0] == 0 || i[0] == m - 1 || i[1] == 0 || i[1] == m - 1 || i[2] == 0 || i[2] == m - 1)) continue;
+    for (int d = 0; d < 3; d++)
+      if (!(std::abs(x[3 * q + d] - a * (2.0 * i[d] / (m - 1) - 1.0)) <= 1e-13 * a)) return false;
+    q++;
+  }
+  return true;
+}
+
 }  // namespace ffmm
 
 using namespace ffmm;
@@ -378,6 +394,52 @@ int ffmm_opcache_put_cube(ffmm_opcache cache, double w_ref, const double *small,
     o.r_up = r_up;
     o.r_dn = r_dn;
     o.nclass = nclass;
+    // even orders with full-rank pseudo-inverses: every point array in orbit order from here on
+    o.sym = false;
+    o.embed_h = cube_embed(o.p);
+    std::vector<double> small_o, large_o, M2M_o, L2L_o, cls_o;
+    std::vector<int32_t> idx_o;
+    std::vector<int8_t> sgn_o;
+    const bool sym = sym_fits(o.p, o.pc, Ns, r_up, r_dn) && on_lattice(small, o.p) && on_lattice(large, o.pc);
+    if (sym) {
+      o.sym_small = sym_orbits(o.p);
+      o.sym_large = sym_orbits(o.pc);
+      const std::vector<int32_t> &ps = o.sym_small, &pl = o.sym_large;
+      std::vector<int32_t> ip(Ns);
+      for (int i = 0; i < Ns; i++) ip[ps[i]] = i;
+      for (int i = 0; i < Ns; i++) small_o.insert(small_o.end(), small + 3 * ps[i], small + 3 * ps[i] + 3);
+      for (int i = 0; i < Nl; i++) large_o.insert(large_o.end(), large + 3 * pl[i], large + 3 * pl[i] + 3);
+      M2M_o.resize((size_t)Ns * NCHILD * Ns);
+      L2L_o.resize(M2M_o.size());
+      cls_o.resize((size_t)nclass * Ns * Ns);
+      for (int c = 0; c < NCHILD; c++)
+        for (int j = 0; j < Ns; j++)
+          for (int i = 0; i < Ns; i++) {
+            M2M_o[((size_t)c * Ns + j) * Ns + i] = M2M[((size_t)c * Ns + ps[j]) * Ns + ps[i]];
+            L2L_o[(size_t)j * NCHILD * Ns + c * Ns + i] = L2L[(size_t)ps[j] * NCHILD * Ns + c * Ns + ps[i]];
+          }
+      for (int c = 0; c < nclass; c++)
+        for (int j = 0; j < Ns; j++)
+          for (int i = 0; i < Ns; i++)
+            cls_o[((size_t)c * Ns + j) * Ns + i] = class_ops[((size_t)c * Ns + ps[j]) * Ns + ps[i]];
+      idx_o.resize((size_t)NFAR * Ns);
+      sgn_o.resize((size_t)NFAR * Ns);
+      for (int f = 0; f < NFAR; f++)
+        for (int i = 0; i < Ns; i++) {
+          const int32_t k = idx[(size_t)f * Ns + ps[i]];
+          if (k < 0 || k >= Ns) fail(FFMM_ERR_ARGUMENT, "idx is not a permutation");
+          idx_o[(size_t)f * Ns + i] = ip[k];
+          sgn_o[(size_t)f * Ns + i] = sgn[(size_t)f * Ns + ps[i]];
+        }
+      std::vector<int32_t> e(Ns);
+      for (int i = 0; i < Ns; i++) e[i] = o.embed_h[ps[i]];
+      o.embed_h = e;
+      small = small_o.data();
+      large = large_o.data();
+      class_ops = cls_o.data();
+      idx = idx_o.data();
+      sgn = sgn_o.data();
+    }
     o.small_h.assign(small, small + 3 * Ns);
     o.large_h.assign(large, large + 3 * Nl);
     std::vector<double> soa(3 * Nl);
@@ -386,38 +448,25 @@ int ffmm_opcache_put_cube(ffmm_opcache cache, double w_ref, const double *small,
     o.large.upload(soa.data(), soa.size(), s);
     std::vector<float> soa32(soa.begin(), soa.end());
     o.large32.upload(soa32.data(), soa32.size(), s);
-    o.Uh_up.upload(Uh_up, (size_t)r_up * Nl, s);
-    std::vector<double> uhp;
-    if (r_up > 240 && r_up <= 304) {
-      const size_t nk = (size_t)(Nl + UC2E_PK - 1) / UC2E_PK * UC2E_PK + 4 * UC2E_PKX;
-      uhp.assign(nk * UC2E_PROWS, 0.0);
-      for (int k = 0; k < Nl; k++)
-        for (int i = 0; i < r_up; i++) uhp[(size_t)k * UC2E_PROWS + i] = Uh_up[(size_t)k * r_up + i];
-      o.Uh_up_pad.upload(uhp.data(), uhp.size(), s);
+    if (sym) {
+      sym_setup(o, small_o, large_o, M2M_o, L2L_o);
+    } else {
+      o.Uh_up.upload(Uh_up, (size_t)r_up * Nl, s);
+      o.Uh_dn.upload(Uh_dn, (size_t)r_dn * Ns, s);
+      std::vector<double> vs((size_t)Ns * r_up);
+      for (int j = 0; j < r_up; j++)
+        for (int i = 0; i < Ns; i++) vs[(size_t)j * Ns + i] = V_up[(size_t)j * Ns + i] * invS_up[j];
+      o.Vs_up.upload(vs.data(), vs.size(), s);
+      std::vector<double> vd((size_t)Nl * r_dn);
+      for (int j = 0; j < r_dn; j++)
+        for (int i = 0; i < Nl; i++) vd[(size_t)j * Nl + i] = V_dn[(size_t)j * Nl + i] * invS_dn[j];
+      o.Vs_dn.upload(vd.data(), vd.size(), s);
+      o.M2M.upload(M2M, (size_t)Ns * NCHILD * Ns, s);
+      std::vector<float> m32(M2M, M2M + (size_t)Ns * NCHILD * Ns);
+      o.M2M32.upload(m32.data(), m32.size(), s);
+      o.L2L.upload(L2L, (size_t)NCHILD * Ns * Ns, s);
+      ctx.sync();   // before the host copies go
     }
-    o.Uh_dn.upload(Uh_dn, (size_t)r_dn * Ns, s);
-    std::vector<double> vs((size_t)Ns * r_up);
-    for (int j = 0; j < r_up; j++)
-      for (int i = 0; i < Ns; i++) vs[(size_t)j * Ns + i] = V_up[(size_t)j * Ns + i] * invS_up[j];
-    o.Vs_up.upload(vs.data(), vs.size(), s);
-    // operand copies of the column GEMMs (rows and k in the kernel's tiles), zero-padded
-    auto pad_rows = [&](DBuf<double> &dst, const double *a, int rows, int K) {
-      const size_t nk = (size_t)(K + UC2E_PK - 1) / UC2E_PK * UC2E_PK + 4 * UC2E_PKX;
-      std::vector<double> ap(nk * UC2E_PROWS, 0.0);
-      for (int k = 0; k < K; k++)
-        for (int i = 0; i < rows; i++) ap[(size_t)k * UC2E_PROWS + i] = a[(size_t)k * rows + i];
-      dst.upload(ap.data(), ap.size(), s);
-    };
-    if (Ns > 240 && Ns <= 304) pad_rows(o.Vs_up_pad, vs.data(), Ns, r_up);
-    if (r_dn > 240 && r_dn <= 304) pad_rows(o.Uh_dn_pad, Uh_dn, r_dn, Ns);
-    std::vector<double> vd((size_t)Nl * r_dn);
-    for (int j = 0; j < r_dn; j++)
-      for (int i = 0; i < Nl; i++) vd[(size_t)j * Nl + i] = V_dn[(size_t)j * Nl + i] * invS_dn[j];
-    o.Vs_dn.upload(vd.data(), vd.size(), s);
-    o.M2M.upload(M2M, (size_t)Ns * NCHILD * Ns, s);
-    std::vector<float> m32(M2M, M2M + (size_t)Ns * NCHILD * Ns);
-    o.M2M32.upload(m32.data(), m32.size(), s);
-    o.L2L.upload(L2L, (size_t)NCHILD * Ns * Ns, s);
     o.class_ops.upload(class_ops, (size_t)nclass * Ns * Ns, s);
     std::vector<float> c32(class_ops, class_ops + (size_t)nclass * Ns * Ns);
     o.class_ops32.upload(c32.data(), c32.size(), s);
@@ -666,6 +715,19 @@ int ffmm_opcache_put_class_factors(ffmm_opcache cache, double tol, const int32_t
     Context &ctx = *o.ctx;
     set_device(ctx);
     hipStream_t s = ctx.stream;
+    std::vector<double> A_o, Bt_o;
+    if (o.sym) {   // the device's orbit order of the surface points
+      A_o.resize(tot);
+      Bt_o.resize(tot);
+      for (int c = 0; c < o.nclass; c++)
+        for (int j = 0; j < f->rank[c]; j++)
+          for (int i = 0; i < o.Ns; i++) {
+            A_o[f->off[c] + (int64_t)j * o.Ns + i] = A[f->off[c] + (int64_t)j * o.Ns + o.sym_small[i]];
+            Bt_o[f->off[c] + (int64_t)i * f->rank[c] + j] = Bt[f->off[c] + (int64_t)o.sym_small[i] * f->rank[c] + j];
+          }
+      A = A_o.data();
+      Bt = Bt_o.data();
+    }
     f->A.upload(A, tot, s);
     f->Bt.upload(Bt, tot, s);
     std::vector<float> a32(A, A + tot), b32(Bt, Bt + tot);
@@ -1422,12 +1484,28 @@ int ffmm_plan_download_expansions(ffmm_plan plan, double *multipoles, double *pl
   return guard([&] {
     if (!plan) fail(FFMM_ERR_ARGUMENT, "null plan");
     Plan &p = plan->c;
+    const OpCache &o = *p.ops;
     set_device(*p.ctx);
     hipStream_t s = p.ctx->stream;
-    if (multipoles) p.Mp.download(multipoles, (size_t)p.ops->Ns * p.nnodes, s);
-    if (plocals) p.Pl.download(plocals, (size_t)p.ops->Ns * p.nnodes, s);
-    if (leaf_locals) p.Lc.download(leaf_locals, (size_t)p.ops->Nl * p.leaf_off[p.L], s);
+    if (multipoles) p.Mp.download(multipoles, (size_t)o.Ns * p.nnodes, s);
+    if (plocals) p.Pl.download(plocals, (size_t)o.Ns * p.nnodes, s);
+    if (leaf_locals) p.Lc.download(leaf_locals, (size_t)o.Nl * p.leaf_off[p.L], s);
     p.ctx->sync();
+    if (!o.sym) return;
+    // from orbit order to the surfaces' own
+    auto unpermute = [](double *a, const std::vector<int32_t> &perm, int64_t n) {
+      if (!a) return;
+      const size_t m = perm.size();
+      std::vector<double> t(m);
+      for (int64_t q = 0; q < n; q++) {
+        double *c = a + (size_t)q * m;
+        for (size_t i = 0; i < m; i++) t[perm[i]] = c[i];
+        std::copy(t.begin(), t.end(), c);
+      }
+    };
+    unpermute(multipoles, o.sym_small, p.nnodes);
+    unpermute(plocals, o.sym_small, p.nnodes);
+    unpermute(leaf_locals, o.sym_large, p.leaf_off[p.L]);
   });
 }
 

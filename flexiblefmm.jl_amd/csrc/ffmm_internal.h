@@ -79,6 +79,14 @@ __device__ __forceinline__ double rsqrt_f64(double x) {
   return y;
 }
 
+// A workgroup barrier that orders LDS accesses only: no wait for the global loads and
+// stores in flight (a prefetch consumed by the same thread, results written out).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // runs upload() once per device and key, under a lock, so that no caller returns
 // before the upload is done (the constant tables, which concurrent plans on other
 // streams read)
@@ -228,7 +236,6 @@ using HTab = HTabT<double>;
 using HTab32 = HTabT<float>;
 
 struct ClassFactors;
-constexpr int UC2E_PROWS = 320, UC2E_PK = 64, UC2E_PKX = 2;   // rows, k rounding, extra k-steps
 
 struct OpCache {
   Context *ctx = nullptr;
@@ -269,12 +276,13 @@ struct OpCache {
   DBuf<double> large;                        // 3 x Nl SoA: x[Nl], y[Nl], z[Nl]
   DBuf<float> large32;
   DBuf<double> Uh_up, Vs_up, Uh_dn, Vs_dn;   // Vs = V diag(invS)
-  // the fused S2M + UC2E kernel's Uh (ranks 241..304): UC2E_PROWS rows per check point,
-  // Nl rounded up to UC2E_PK and UC2E_PKX k-steps more, zero-padded (no guards on its loads)
-  DBuf<double> Uh_up_pad;
-  // the column GEMMs' operators (k_gemm_cols: UC2E's V diag(invS), DC2E's Uh), the same
-  // layout (UC2E_PROWS rows per k, k rounded up to UC2E_PK and UC2E_PKX k-steps more)
-  DBuf<double> Vs_up_pad, Uh_dn_pad;
+  // even orders with full-rank pseudo-inverses (sym.hip): the surfaces in orbit order
+  // (sym_small, sym_large: device point -> given point), the operators' 8 symmetric blocks
+  // (k-major, rows padded to 16, k to sym_kp / sym_kp2): UC2E's factors, DC2E's factors, M2M, L2L
+  bool sym = false;
+  int sym_kp = 0, sym_kp2 = 0;
+  std::vector<int32_t> sym_small, sym_large;
+  DBuf<double> sym_rep, sym_u1, sym_u2, sym_d1, sym_d2, sym_m2m, sym_l2l;
   DBuf<double> M2M, L2L, class_ops;
   DBuf<float> M2M32, class_ops32;   // FP32 copies for the mixed form
   DBuf<int32_t> far_class, idx, inv;         // idx/inv: [f * Ns + i]
@@ -365,7 +373,7 @@ struct Plan {
   // work buffers
   DBuf<double> pM, tup, Mup, tM, G, tdn, Gc, Yc;
   DBuf<float> Gc32, Yc32, pM32;
-  DBuf<float> Mp32, tM32;  // the cube's mixed M2M: an FP32 mirror of Mp (written beside it), the parents' products
+  DBuf<float> Mp32, tM32;  // the dense mixed M2M: an FP32 mirror of Mp (written beside it), the parents' products
   // spectral M2L workspace
   DBuf<double> spec_S, spec_U;
   DBuf<float> spec_S32, spec_U32;
@@ -464,6 +472,21 @@ void spectral_prepare(Plan &plan);
 void spectral_workspace(Plan &plan);
 bool spectral_tile_counts(const Plan &plan, int l, int64_t &staged, int64_t &per_group);
 void m2l_spectral_level(Plan &plan, int l);
+
+// ---- the cube method's translations by symmetric blocks (sym.hip) ----
+std::vector<int32_t> sym_orbits(int n);
+bool sym_fits(int p, int pc, int Ns, int r_up, int r_dn);
+void sym_setup(OpCache &o, const std::vector<double> &small, const std::vector<double> &large,
+               const std::vector<double> &M2M, const std::vector<double> &L2L);
+// fewer childless sourced nodes than this: S2M as a kernel of its own (a workgroup per node
+// and 64 orbits), else inside UC2E (16 nodes per workgroup)
+constexpr int64_t SYM_SPLIT_NODES = 8192;
+bool sym_split_s2m(int64_t nq);
+void sym_s2m_uc2e(Plan &plan, const int32_t *nodes, int64_t nq);
+void sym_m2m(Plan &plan, int l);
+void sym_l2l(Plan &plan, int l);
+void sym_dc2e(Plan &plan, const int32_t *leaves, int64_t nq, double *Lc);
+void sym_zero_unsourced(Plan &plan);
 
 // ---- direct sums (direct.hip) ----
 void direct(Context &ctx, const double *src, const double *tau, int64_t ns, const double *tgt, int64_t nt,

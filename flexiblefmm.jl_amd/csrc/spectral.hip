@@ -636,14 +636,6 @@ __device__ __forceinline__ void hu_store(float2 *Us, int t, const float4 v[HU_NV
   }
 }
 
-// A workgroup barrier that orders LDS accesses only: no wait for the global loads and
-// stores in flight (a prefetch consumed by the same thread, results written out).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // two workgroups per CU (8 waves each): 4 waves per SIMD, at most 128 VGPRs
 __global__ void __launch_bounds__(HU_TB) __attribute__((amdgpu_waves_per_eu(4, 4))) k_spec_hadamard_union(
     const float2 *__restrict__ S, float2 *__restrict__ U, const float2 *__restrict__ tables,

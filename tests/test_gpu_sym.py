@@ -1,0 +1,58 @@
+"""The cube method's translations by symmetric blocks (csrc/sym.hip) against the oracle's
+dense operators on the same tree: every even order the kernels take (1, 7, 19, 37 and 61
+orbits: one to four row tiles, full and ragged), S2M as its own kernel and inside UC2E, both
+precisions, workgroups with missing columns; an odd order keeps the dense operators."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+BOX = (np.zeros(3), 1.0)
+
+
+@pytest.mark.parametrize("p,n,ppl,precision", [
+    (2, 1500, 20, "f64"), (4, 3000, 20, "f64"), (5, 2000, 25, "f64"), (6, 3001, 30, "f64"), (8, 2500, 25, "f64"),
+    (10, 2000, 40, "f64"), (4, 3000, 20, "mixed"), (6, 3001, 30, "mixed"), (8, 2500, 25, "mixed"),
+    (4, 40_000, 4, "f64"), (6, 40_000, 4, "mixed")])
+def test_blocks_vs_oracle(p, n, ppl, precision):
+    """FP64: the oracle's rounding, 1e-11 (1e-10 at p = 10, whose pseudo-inverses are ten
+    times worse conditioned); mixed: the FP32 M2L and evaluation, 2e-6."""
+    import ffmm
+    print(f"[sym] p={p} n={n} ppl={ppl} {precision}", flush=True)
+    rng = np.random.default_rng(100 * p + ppl)
+    pts = rng.random((n, 3))
+    pts[: n // 3] = 0.4 + 0.05 * rng.random((n // 3, 3))
+    tau = rng.standard_normal(n)
+    m = ffmm.CubeKernelIndependent(ffmm.Laplace3D(), p=p)
+    cache = ffmm.OperatorCache(m)
+    plan = ffmm.DevicePlan(m, pts, ppl=ppl, bbox=BOX, cache=cache, precision=precision)
+    u = plan.matvec(tau).cpu().numpy()
+    ref = O.FMM(cache.host_operators(), pts, ppl, BOX[0], BOX[1])
+    u_ref = ref.matvec(tau)
+    split = int(plan.level_s2m[2:].sum()) < 8192
+    assert split == (n < 40_000)             # both forms of S2M are covered
+    if precision == "mixed":
+        assert np.linalg.norm(u - u_ref) < 2e-6 * np.linalg.norm(u_ref)
+    else:
+        assert np.max(np.abs(u - u_ref)) < (1e-10 if p == 10 else 1e-11) * np.max(np.abs(u_ref))
+
+
+@pytest.mark.parametrize("precision", ["f64", "mixed"])
+def test_sources_beyond_the_lds_stage(precision):
+    """1,350,000 uniform points with ppl = 110: the 32,768 boxes of level 5 are leaves of ~41
+    sources, so workgroups of 16 of them hold more sources than the fused kernel stages in
+    LDS (320 in FP64, 640 in FP32) and read them from global memory."""
+    import ffmm
+    n = 1_350_000
+    print(f"[sym] heavy nodes {precision}", flush=True)
+    rng = np.random.default_rng(5)
+    pts, tau = rng.random((n, 3)), rng.standard_normal(n)
+    m = ffmm.CubeKernelIndependent(ffmm.Laplace3D(), p=4)
+    cache = ffmm.OperatorCache(m)
+    plan = ffmm.DevicePlan(m, pts, ppl=110, bbox=BOX, cache=cache, precision=precision)
+    assert int(plan.level_s2m[2:].sum()) >= 8192 and plan.N / int(plan.level_s2m.sum()) > 40
+    u = plan.matvec(tau).cpu().numpy()
+    u_ref = O.FMM(cache.host_operators(), pts, 110, BOX[0], BOX[1]).matvec(tau)
+    assert np.linalg.norm(u - u_ref) < (2e-6 if precision == "mixed" else 1e-11) * np.linalg.norm(u_ref)
