@@ -519,13 +519,7 @@ int ffmm_opcache_put_cube(ffmm_opcache cache, double w_ref, const double *small,
       ctx.sync();
     }
     o.has_tables = tables != nullptr;
-    if (tables) {
-      const int n = 2 * o.p;
-      const size_t nfreq = (size_t)n * n * (o.p + 1);
-      o.tables.upload(tables, 2 * nfreq * NFAR, s);
-      std::vector<float> t32(tables, tables + 2 * nfreq * NFAR);
-      o.tables32.upload(t32.data(), t32.size(), s);
-    }
+    if (tables) spectral_setup(o, tables);
     ctx.sync();
     o.ready = true;
   });

@@ -292,8 +292,9 @@ struct OpCache {
   // fsel[f, i] = the target-frame position j of product entry i (inv[f, j] = i), sign sgn_t[f, i]
   DBuf<int32_t> fsel;
   DBuf<int8_t> sgn;
-  DBuf<double> tables;                       // 316 x nfreq complex (interleaved)
-  DBuf<float> tables32;
+  // the spectral M2L's table operands (spectral.hip: k_had_fragments), bfloat16 and FP64
+  DBuf<uint16_t> had_mixed;
+  DBuf<double> had_f64, had_zero;
   DBuf<int32_t> embed;                       // Ns: lattice index of each small-surface point
   DBuf<int32_t> sub8;                        // Ns: its index in the p^3 corner of the lattice
   DBuf<int16_t> lat8;                        // p^3: the surface point at a corner lattice index, or -1
@@ -377,14 +378,12 @@ struct Plan {
   // spectral M2L workspace
   DBuf<double> spec_S, spec_U;
   DBuf<float> spec_S32, spec_U32;
-  std::vector<DBuf<int32_t>> spec_gptr, spec_cand;   // per level: sibling groups' far-source candidates (FP64)
-  std::vector<DBuf<int32_t>> spec_gcol, spec_tiles;  // per level: groups' colleague children, active tiles (FP32)
-  std::vector<int64_t> spec_ntiles;
-  // per level and active tile: its sourced colleagues staged together (the boxes by
-  // staging row, each (group, colleague)'s row); the tiles that fit and those that do not
-  std::vector<DBuf<int32_t>> spec_ulist, spec_fit, spec_over;
-  std::vector<DBuf<uint8_t>> spec_uslot;
-  std::vector<int64_t> spec_nfit, spec_nover;
+  // the tiles of 16 sibling groups of all levels: each subtile's staged boxes and slots, its
+  // part of the tile (0: none); the subtiles in order; per level their number, the first one
+  // and the level's first tile
+  DBuf<int32_t> spec_ulist, spec_subs;
+  DBuf<uint8_t> spec_uslot, spec_flag;
+  std::vector<int64_t> spec_nsub, spec_sub0, spec_tile0;
   // targets
   DBuf<double> tgt_sorted;
   DBuf<int32_t> tgt_node, tgt_leafslot, tgt_order, tgt_ptr;
@@ -467,10 +466,11 @@ void gather_inputs(Plan &plan, const double *tau, int sorted);
 void upward_pass(Plan &plan);
 void downward_pass(Plan &plan);
 void m2l_dense_level(Plan &plan, int l);
+void spectral_setup(OpCache &o, const double *tables);
 void spectral_prepare(Plan &plan);
 // the spectra of one level's sources and targets (the largest level's size)
 void spectral_workspace(Plan &plan);
-bool spectral_tile_counts(const Plan &plan, int l, int64_t &staged, int64_t &per_group);
+bool spectral_tile_counts(const Plan &plan, int l, int64_t &staged, int64_t &cut);
 void m2l_spectral_level(Plan &plan, int l);
 
 // ---- the cube method's translations by symmetric blocks (sym.hip) ----

@@ -61,13 +61,7 @@ size_t plan_bytes(const Plan &p) {
        cap_bytes(p.Gc) + cap_bytes(p.Yc) + cap_bytes(p.Gc32) + cap_bytes(p.Yc32) + cap_bytes(p.pM32) + cap_bytes(p.Mp32) + cap_bytes(p.tM32);
   s += cap_bytes(p.spec_S) + cap_bytes(p.spec_U) + cap_bytes(p.spec_S32) + cap_bytes(p.spec_U32);
   s += cap_bytes(p.Zc) + cap_bytes(p.Zc32) + cap_bytes(p.gin) + cap_bytes(p.gout);
-  for (const auto &b : p.spec_gptr) s += cap_bytes(b);
-  for (const auto &b : p.spec_cand) s += cap_bytes(b);
-  for (const auto &b : p.spec_gcol) s += cap_bytes(b);
-  for (const auto &b : p.spec_tiles) s += cap_bytes(b);
-  for (const auto *v : {&p.spec_ulist, &p.spec_fit, &p.spec_over})
-    for (const auto &b : *v) s += cap_bytes(b);
-  for (const auto &b : p.spec_uslot) s += cap_bytes(b);
+  s += cap_bytes(p.spec_ulist) + cap_bytes(p.spec_subs) + cap_bytes(p.spec_uslot) + cap_bytes(p.spec_flag);
   s += cap_bytes(p.tgt_sorted) + cap_bytes(p.tgt_node) + cap_bytes(p.tgt_leafslot) + cap_bytes(p.tgt_order) +
        cap_bytes(p.tgt_ptr) + cap_bytes(p.tgt_keys);
   return s;
@@ -82,7 +76,7 @@ static int64_t estimate_bytes(const OpCache &o, int64_t n, int ppl, int m2l, int
   const double nodes = 12.0 * (double)n / ppl + 64, leaves = 5.0 * (double)n / ppl + 64;
   double b = nodes * (2.0 * o.Ns * 8) + leaves * (o.Nl * 8.0) + 256.0 * n + 96.0 * nt;
   if (o.method == METHOD_CUBE) b += leaves * (o.Nl + 3.0 * o.Ns) * 8;
-  if (m2l == FFMM_M2L_SPECTRAL) b += 0.6 * nodes * 2304 * 16;
+  if (m2l == FFMM_M2L_SPECTRAL) b += 0.6 * nodes * 1688 * 16;
   // dense class M2L: the class-major pair table, and the gathered columns and products of
   // one target chunk (at most about 2 GiB)
   if (m2l == FFMM_M2L_DENSE) b += 4.0 * o.nclass * nodes + std::min<double>(2.2e9, 2.0 * o.Ns * 8 * 200.0 * nodes);
