@@ -580,6 +580,7 @@ int ffmm_opcache_create_harmonic(ffmm_context ctx, int kernel, int p, double kap
       }
     }
     o.offs.upload(offs.data(), offs.size(), ctx->c.stream);
+    sym_harmonic_entries(o);
     ctx->c.sync();
     *out = h.release();
   });
@@ -640,7 +641,10 @@ int ffmm_opcache_put_harmonic_level(ffmm_opcache cache, double width, const doub
     const int N = o.hN, NB = o.Ns;
     auto lv = std::make_unique<HarmonicLevel>();
     lv->w = width;
-    if (o.nb == 1) {
+    sym_harmonic_setup(o, *lv, M2M, L2L);
+    if (lv->sym_m2m.p) {
+      // by blocks: the dense forms are not needed
+    } else if (o.nb == 1) {
       lv->M2M.upload(M2M, (size_t)N * NCHILD * N, s);
       lv->L2L.upload(L2L, (size_t)NCHILD * N * N, s);
     } else {

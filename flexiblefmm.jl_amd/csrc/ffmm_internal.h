@@ -219,7 +219,10 @@ constexpr int METHOD_HARMONIC = 1;   // SphericalHarmonics (Laplace3D, Yukawa3D)
 // the operators of the harmonic methods for boxes of one width
 struct HarmonicLevel {
   double w = 0.0;
-  DBuf<double> M2M, L2L;   // NB x 8NB, 8NB x NB (NB = nb N; the dense Stokes forms for nb = 4)
+  // the blocks of M2M and L2L by reflection parity (sym.hip), or, where the scalar operators
+  // do not split (sym_m2m empty), NB x 8NB and 8NB x NB (NB = nb N; dense Stokes forms for nb = 4)
+  DBuf<double> sym_m2m, sym_l2l;
+  DBuf<double> M2M, L2L;
   DBuf<double> reps;       // nclass x (N x N)
   DBuf<float> reps32;      // the same in FP32 (the mixed form's M2L)
   DBuf<float> reps32r;     // FP32, row-major, zero-padded to 128 x 128 per class (N <= 128: the fused mixed M2L)
@@ -248,6 +251,9 @@ struct OpCache {
   bool has_classes = false;
   DBuf<double> htab;                         // a, b, cz, cm, cp (ntri each), e (p)
   DBuf<float> htab32;                        // the same, rounded to FP32
+  DBuf<uint8_t> hchi, hrank;                 // each entry's reflection block and its place there
+  std::vector<uint8_t> hchi_h, hrank_h;
+  int hmax = 0;                              // entries of the largest block
   DBuf<int8_t> sgn_t;                        // target-side signs [f * N + i] (the cube: = sgn)
   DBuf<double> offs;                         // 316 x 3 far offsets (the Stokes coupling)
   // the operators by width; entries are added, never replaced or removed while the
@@ -487,6 +493,10 @@ void sym_m2m(Plan &plan, int l);
 void sym_l2l(Plan &plan, int l);
 void sym_dc2e(Plan &plan, const int32_t *leaves, int64_t nq, double *Lc);
 void sym_zero_unsourced(Plan &plan);
+void sym_harmonic_entries(OpCache &o);
+void sym_harmonic_setup(OpCache &o, HarmonicLevel &lv, const double *M2M, const double *L2L);
+void sym_harmonic_m2m(Plan &plan, int l);
+void sym_harmonic_l2l(Plan &plan, int l);
 
 // ---- direct sums (direct.hip) ----
 void direct(Context &ctx, const double *src, const double *tau, int64_t ns, const double *tgt, int64_t nt,

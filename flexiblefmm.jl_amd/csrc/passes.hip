@@ -709,12 +709,31 @@ void upward_pass(Plan &plan) {
   const int l2 = std::min(2, plan.L);
   const int64_t nq = plan.s2m_off[plan.L] - plan.s2m_off[l2];
   const int32_t *nodes = plan.s2m_nodes.p + plan.s2m_off[l2];
-  if (o.sym) {
+  const bool harm = o.method == METHOD_HARMONIC;
+  if (o.sym || harm) {
     // every sourced column from level 2 down is written before it is read; the others are zero
     const int64_t n01 = l2 < plan.L ? plan.lo[l2] : plan.nnodes;
     k_fill<<<nblocks((int64_t)Ns * n01, TB), TB, 0, s>>>(plan.Mp.p, (int64_t)Ns * n01, 0.0);
     FFMM_LAUNCH_CHECK();
     sym_zero_unsourced(plan);
+    if (harm) {
+      for (int l = plan.L - 1; l >= 2; l--) {
+        // the multipoles directly (partial_to_multipole! is a copy, src/operators/harmonics.jl:441)
+        harmonic_s2m_level(plan, l);
+        if (l == plan.L - 1) continue;
+        if (plan.hl[l]->sym_m2m.p) {
+          sym_harmonic_m2m(plan, l);
+          continue;
+        }
+        const int64_t ng = plan.nl[l + 1] / NCHILD;
+        gemm(ctx, Ns, (int)ng, NCHILD * Ns, 1.0, plan.hl[l]->M2M.p, Ns, plan.Mp.p + plan.lo[l + 1] * Ns, NCHILD * Ns, 0.0,
+             plan.tM.p, Ns);
+        k_scatter_parents<double><<<nblocks((int64_t)Ns * ng, TB), TB, 0, s>>>(plan.Mp.p, plan.tM.p, plan.parent.p,
+                                                                               plan.lo[l + 1], Ns, ng, 1.0, nullptr);
+        FFMM_LAUNCH_CHECK();
+      }
+      return;
+    }
     if (nq > 0) sym_s2m_uc2e(plan, nodes, nq);
     for (int l = plan.L - 2; l >= 2; l--) sym_m2m(plan, l);
     return;
@@ -722,7 +741,7 @@ void upward_pass(Plan &plan) {
   // every column is written before it is read except by M2M of empty groups: clear.  The
   // cube's mixed form keeps an FP32 mirror of the multipoles, written beside them by the
   // UC2E and M2M scatters, that its FP32 M2M GEMMs read directly
-  const bool mirror = o.method == METHOD_CUBE && plan.precision == FFMM_PREC_MIXED;
+  const bool mirror = plan.precision == FFMM_PREC_MIXED;
   float *Mp32 = mirror ? plan.Mp32.p : nullptr;
   k_fill<<<nblocks(plan.Mp.n, TB), TB, 0, s>>>(plan.Mp.p, plan.Mp.n, 0.0);
   FFMM_LAUNCH_CHECK();
@@ -730,7 +749,7 @@ void upward_pass(Plan &plan) {
     k_fill32<<<nblocks(plan.Mp32.n, TB), TB, 0, s>>>(Mp32, plan.Mp32.n);
     FFMM_LAUNCH_CHECK();
   }
-  if (o.method == METHOD_CUBE && nq > 0) {
+  if (nq > 0) {
     // the childless sourced nodes of all levels at once (each node's width from its level):
     // S2M into check potentials, then UC2E, M = pinv_scale V diag(invS) (Uh pM)
     // (src/device_passes.jl:496-502), as two GEMMs over all of them.  pinv_scale = lam[l]
@@ -751,14 +770,9 @@ void upward_pass(Plan &plan) {
     FFMM_LAUNCH_CHECK();
   }
   for (int l = plan.L - 1; l >= 2; l--) {
-    if (o.method == METHOD_HARMONIC) {
-      // the multipoles directly (partial_to_multipole! is a copy, src/operators/harmonics.jl:441)
-      harmonic_s2m_level(plan, l);
-    }
     if (l < plan.L - 1) {
       const int64_t ng = plan.nl[l + 1] / NCHILD;
       const double *B = plan.Mp.p + plan.lo[l + 1] * Ns;
-      const double *M2M = o.method == METHOD_HARMONIC ? plan.hl[l]->M2M.p : o.M2M.p;
       if (mirror) {
         // the mixed form: M2M as an FP32 GEMM over the children's FP32 mirror (its rounding
         // is not amplified: the multipoles feed M2L, never a pseudo-inverse).  Wide levels
@@ -774,7 +788,7 @@ void upward_pass(Plan &plan) {
         k_scatter_parents<float><<<nblocks((int64_t)Ns * ng, TB), TB, 0, s>>>(plan.Mp.p, plan.tM32.p, plan.parent.p,
                                                                               plan.lo[l + 1], Ns, ng, 1.0, Mp32);
       } else {
-        gemm(ctx, Ns, (int)ng, NCHILD * Ns, 1.0, M2M, Ns, B, NCHILD * Ns, 0.0, plan.tM.p, Ns);
+        gemm(ctx, Ns, (int)ng, NCHILD * Ns, 1.0, o.M2M.p, Ns, B, NCHILD * Ns, 0.0, plan.tM.p, Ns);
         k_scatter_parents<double><<<nblocks((int64_t)Ns * ng, TB), TB, 0, s>>>(plan.Mp.p, plan.tM.p, plan.parent.p,
                                                                                plan.lo[l + 1], Ns, ng, 1.0, nullptr);
       }
@@ -895,6 +909,8 @@ void downward_pass(Plan &plan) {
     double *pL = plan.Pl.p + plan.lo[l] * Ns;
     if (l > 2 && o.sym) {
       sym_l2l(plan, l);
+    } else if (l > 2 && o.method == METHOD_HARMONIC && plan.hl[l - 1]->sym_l2l.p) {
+      sym_harmonic_l2l(plan, l);
     } else if (l > 2) {
       k_gather_parents<<<nblocks((int64_t)Ns * ng, TB), TB, 0, s>>>(plan.G.p, plan.Pl.p, plan.parent.p, plan.lo[l],
                                                                     Ns, ng);

@@ -1,4 +1,4 @@
-// The cube method's translations in the reflection symmetry of the cube.
+// The translations of the cube and the harmonic methods in the reflection symmetry of the cube.
 //
 // The surfaces of a box are lattices that the three reflections x -> -x, y -> -y, z -> -z
 // map onto themselves, and the Laplace kernel is invariant under them.  With an even
@@ -511,6 +511,183 @@ __global__ void __launch_bounds__(SY_TB, 4) k_sym_down(SyDown a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// The harmonic methods: a solid harmonic has a parity under each reflection, so entry i of
+// an expansion belongs to one block chi_i, and the translation of child c is that of child 0
+// with signs, A_c[i, j] = chi_i(c) chi_j(c) A_0[i, j].  So M2M is
+//   out_i = sum_j A_0[i, j] W[chi_i ^ chi_j, j],  W[psi, j] = sum_c (-1)^popcount(psi & c) m_(c, j)
+// (block chi: its rows of A_0 against N transformed entries), and L2L
+//   y_(c, i) = chi_i(c) sum_psi (-1)^popcount(psi & c) sum_(j in psi) B_0[i, j] l_j:
+// N^2 products per column where the dense forms take 8 N^2 (Stokes: 128 N^2 per 4 columns).
+// Stokes: the four blocks are columns of the same operator; the coupling of the fourth with
+// the child's offset d is applied to the children before M2M (m_4 / 2 + d . m) and to the
+// children after L2L (2 y_4 - 2 d . y) (src/operators/harmonics_stokes.jl:112-131).
+// 16 columns per workgroup: 16 groups, or 4 groups of 4 blocks.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ double child_offset(int c, int a) { return (c >> a) & 1 ? 0.25 : -0.25; }
+
+template <int RT, int NB>
+__global__ void __launch_bounds__(SY_TB, 4) k_harm_m2m(const double *__restrict__ B, int N, int KP,
+                                                       const uint8_t *__restrict__ chi,
+                                                       const uint8_t *__restrict__ rank,
+                                                       const int32_t *__restrict__ parent,
+                                                       const uint8_t *__restrict__ has_source, int64_t first, int64_t ng,
+                                                       double *__restrict__ Mp) {
+  constexpr int R = 16 * RT, G = SY_N / NB;
+  __shared__ double P[8][SY_K * SY_S];
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int li = lane & 15, lk = lane >> 4;
+  const int64_t g0 = (int64_t)blockIdx.x * G;
+  sy_f64x4 acc[RT];
+#pragma unroll
+  for (int i = 0; i < RT; i++) acc[i] = sy_f64x4{0.0, 0.0, 0.0, 0.0};
+  const double *A = B + ((size_t)w * KP + lk) * R + li;
+  for (int k0 = 0; k0 < N; k0 += SY_K) {
+    const int j = k0 + lane;
+    const int cj = j < N ? chi[j] : 0;
+    if (k0 > 0) lds_barrier();
+    auto put = [&](double v[8], int col) {
+      wht8(v);
+#pragma unroll
+      for (int h = 0; h < 8; h++) P[h ^ cj][lane * SY_S + col] = v[h];
+    };
+    auto get = [&](int64_t g, int b, double v[8]) {
+#pragma unroll
+      for (int c = 0; c < 8; c++) {
+        const int64_t node = first + NCHILD * g + c;
+        v[c] = g < ng && j < N && has_source[node] ? Mp[(node * NB + b) * N + j] : 0.0;
+      }
+    };
+    if constexpr (NB == 1) {
+#pragma unroll
+      for (int m = 0; m < 2; m++) {
+        double v[8];
+        get(g0 + w + 8 * m, 0, v);
+        put(v, w + 8 * m);
+      }
+    } else {   // wave w: group w % 4, its blocks 0, 1 or 2, 3
+      const int gl = w & 3;
+      double v[8], u[8];
+      get(g0 + gl, 0, v);
+      if (w < 4) {
+        put(v, 4 * gl);
+        get(g0 + gl, 1, v);
+        put(v, 4 * gl + 1);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 8; c++) u[c] = child_offset(c, 0) * v[c];
+        get(g0 + gl, 1, v);
+#pragma unroll
+        for (int c = 0; c < 8; c++) u[c] = fma(child_offset(c, 1), v[c], u[c]);
+        get(g0 + gl, 2, v);
+#pragma unroll
+        for (int c = 0; c < 8; c++) u[c] = fma(child_offset(c, 2), v[c], u[c]);
+        put(v, 4 * gl + 2);
+        get(g0 + gl, 3, v);
+#pragma unroll
+        for (int c = 0; c < 8; c++) u[c] = fma(0.5, v[c], u[c]);
+        put(u, 4 * gl + 3);
+      }
+    }
+    lds_barrier();
+    mma_chunk<RT>(acc, A + (size_t)k0 * R, P[w], (min(SY_K, N - k0) + 15) / 16, lk, li);
+  }
+  wave_lds_fence();
+  put_rows<RT>(P[w], acc, lk, li);
+  lds_barrier();
+  for (int e = t; e < SY_N * N; e += SY_TB) {
+    const int col = e / N, i = e % N;
+    const int64_t g = g0 + col / NB;
+    if (g < ng) Mp[((int64_t)parent[first + NCHILD * g] * NB + col % NB) * N + i] = P[chi[i]][rank[i] * SY_S + col];
+  }
+}
+
+template <int RT, int NB>
+__global__ void __launch_bounds__(SY_TB, 4) k_harm_l2l(const double *__restrict__ B, int N, int RP,
+                                                       const uint8_t *__restrict__ chi,
+                                                       const uint8_t *__restrict__ rank,
+                                                       const int32_t *__restrict__ parent, int64_t first, int64_t ng,
+                                                       double *__restrict__ Pl) {
+  constexpr int G = SY_N / NB, KS = 4 * RT;
+  __shared__ double P[8][SY_K * SY_S];
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int li = lane & 15, lk = lane >> 4;
+  const int64_t g0 = (int64_t)blockIdx.x * G;
+  for (int i = lane; i < 4 * KS * SY_S; i += 64) P[w][i] = 0.0;
+  lds_barrier();
+  for (int e = t; e < SY_N * N; e += SY_TB) {
+    const int col = e / N, i = e % N;
+    const int64_t g = g0 + col / NB;
+    if (g < ng)
+      P[chi[i]][rank[i] * SY_S + col] = Pl[((int64_t)parent[first + NCHILD * g] * NB + col % NB) * N + i];
+  }
+  lds_barrier();
+  double b[KS];
+#pragma unroll
+  for (int s = 0; s < KS; s++) b[s] = P[w][(4 * s + lk) * SY_S + li];
+  wave_lds_fence();
+  const double *A = B + ((size_t)w * 4 * KS + lk) * RP + li;
+  for (int k0 = 0; k0 < N; k0 += SY_K) {
+    sy_f64x4 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[i] = sy_f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < KS; s++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) acc[i] = mma(A[(size_t)4 * s * RP + k0 + 16 * i], b[s], acc[i]);
+    if (k0 > 0) lds_barrier();
+    put_rows<4>(P[w], acc, lk, li);
+    lds_barrier();
+    const int i = k0 + lane;
+    const int ci = i < N ? chi[i] : 0;
+    auto get = [&](int col, double v[8]) {   // the 8 children's values of a column
+#pragma unroll
+      for (int h = 0; h < 8; h++) v[h] = P[h][lane * SY_S + col];
+      wht8(v);
+#pragma unroll
+      for (int c = 0; c < 8; c++) v[c] = __builtin_popcount(ci & c) & 1 ? -v[c] : v[c];
+    };
+    auto put = [&](int64_t g, int bl, const double v[8]) {
+      if (g >= ng || i >= N) return;
+#pragma unroll
+      for (int c = 0; c < 8; c++) Pl[((first + NCHILD * g + c) * NB + bl) * N + i] = v[c];
+    };
+    if constexpr (NB == 1) {
+#pragma unroll
+      for (int m = 0; m < 2; m++) {
+        double v[8];
+        get(w + 8 * m, v);
+        put(g0 + w + 8 * m, 0, v);
+      }
+    } else {
+      const int gl = w & 3;
+      double v[8], u[8];
+      get(4 * gl, v);
+      if (w < 4) {
+        put(g0 + gl, 0, v);
+        get(4 * gl + 1, v);
+        put(g0 + gl, 1, v);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 8; c++) u[c] = -2.0 * child_offset(c, 0) * v[c];
+        get(4 * gl + 1, v);
+#pragma unroll
+        for (int c = 0; c < 8; c++) u[c] = fma(-2.0 * child_offset(c, 1), v[c], u[c]);
+        get(4 * gl + 2, v);
+#pragma unroll
+        for (int c = 0; c < 8; c++) u[c] = fma(-2.0 * child_offset(c, 2), v[c], u[c]);
+        put(g0 + gl, 2, v);
+        get(4 * gl + 3, v);
+#pragma unroll
+        for (int c = 0; c < 8; c++) u[c] = fma(2.0, v[c], u[c]);
+        put(g0 + gl, 3, u);
+      }
+    }
+  }
+}
+
 // the columns of nodes without sources are zero (nothing writes them)
 __global__ void k_sym_zero(const uint8_t *__restrict__ has_source, int64_t nn, int Ns, double *__restrict__ Mp) {
   const int lane = threadIdx.x & 63;
@@ -669,6 +846,57 @@ void sym_setup(OpCache &o, const std::vector<double> &small, const std::vector<d
   o.sym = true;
 }
 
+// The block of each entry of a harmonic expansion of degree p (entry n^2 for order 0, n^2 +
+// 2 m - 1 and n^2 + 2 m for the parts of order m: cos and sin) and its place in the block.
+void sym_harmonic_entries(OpCache &o) {
+  std::vector<uint8_t> chi, rank;
+  int cnt[8] = {};
+  for (int n = 0; n <= o.p; n++)
+    for (int k = 0; k < 2 * n + 1; k++) {
+      const int m = (k + 1) / 2, sn = k > 0 && k % 2 == 0;   // sin: even under y -> -y it is not
+      const int c = ((m + sn) & 1) | sn << 1 | ((n + m) & 1) << 2;
+      chi.push_back((uint8_t)c);
+      rank.push_back((uint8_t)cnt[c]++);
+    }
+  o.hmax = *std::max_element(cnt, cnt + 8);
+  if (o.hmax > 64) return;      // more rows than the kernels take: the dense operators
+  o.hchi_h = chi;
+  o.hrank_h = rank;
+  o.hchi.upload(chi.data(), chi.size(), o.ctx->stream);
+  o.hrank.upload(rank.data(), rank.size(), o.ctx->stream);
+}
+
+// The blocks of a width's scalar M2M (N x 8 N) and L2L (8 N x N, column major), the mean
+// over the children; left unset (the dense operators stay) when they are not symmetric.
+void sym_harmonic_setup(OpCache &o, HarmonicLevel &lv, const double *M2M, const double *L2L) {
+  if (o.hmax > 64) return;
+  const int N = o.hN, R = (o.hmax + 15) / 16 * 16, KP = (N + SY_K - 1) / SY_K * SY_K;
+  const std::vector<uint8_t> &chi = o.hchi_h, &rank = o.hrank_h;
+  std::vector<double> mm(8 * (size_t)KP * R + 16 * R, 0.0), ll(8 * (size_t)R * KP, 0.0);
+  double big[2] = {0.0, 0.0}, off[2] = {0.0, 0.0};
+  for (int j = 0; j < N; j++)
+    for (int i = 0; i < N; i++) {
+      double a[2] = {0.0, 0.0}, x[2][8];
+      for (int c = 0; c < NCHILD; c++) {
+        const double s = chi_sign(chi[i] ^ chi[j], c);
+        x[0][c] = s * M2M[((size_t)c * N + j) * N + i];
+        x[1][c] = s * L2L[(size_t)j * NCHILD * N + c * N + i];
+        for (int k = 0; k < 2; k++) a[k] += x[k][c] / 8.0;
+      }
+      for (int k = 0; k < 2; k++)
+        for (int c = 0; c < NCHILD; c++) {
+          big[k] = std::max(big[k], std::abs(x[k][c]));
+          off[k] = std::max(off[k], std::abs(x[k][c] - a[k]));
+        }
+      mm[((size_t)chi[i] * KP + j) * R + rank[i]] = a[0];
+      ll[((size_t)chi[j] * R + rank[j]) * KP + i] = a[1];
+    }
+  if (!(off[0] <= 1e-11 * big[0] && off[1] <= 1e-11 * big[1])) return;
+  lv.sym_m2m.upload(mm.data(), mm.size(), o.ctx->stream);
+  lv.sym_l2l.upload(ll.data(), ll.size(), o.ctx->stream);
+  o.ctx->sync();
+}
+
 // ---------------------------------------------------------------------------
 // the passes' launches
 // ---------------------------------------------------------------------------
@@ -742,6 +970,43 @@ void sym_dc2e(Plan &plan, const int32_t *leaves, int64_t nq, double *Lc) {
                  plan.lam_d.p, plan.Pl.p,  Lc};
   with_nr(o.Ns / 8, [&](auto NR) {
     k_sym_down<1, decltype(NR)::value><<<sy_blocks(nq), SY_TB, 0, plan.ctx->stream>>>(a);
+  });
+  FFMM_LAUNCH_CHECK();
+}
+
+template <class F>
+static void with_harmonic(const OpCache &o, F &&f) {
+  const int rt = (o.hmax + 15) / 16;
+  auto go = [&](auto RT) {
+    if (o.nb == 4) f(RT, std::integral_constant<int, 4>{});
+    else f(RT, std::integral_constant<int, 1>{});
+  };
+  if (rt == 1) go(std::integral_constant<int, 1>{});
+  else if (rt == 2) go(std::integral_constant<int, 2>{});
+  else if (rt == 3) go(std::integral_constant<int, 3>{});
+  else go(std::integral_constant<int, 4>{});
+}
+
+void sym_harmonic_m2m(Plan &plan, int l) {
+  OpCache &o = *plan.ops;
+  const int64_t first = plan.lo[l + 1], ng = plan.nl[l + 1] / NCHILD;
+  const int KP = (o.hN + SY_K - 1) / SY_K * SY_K;
+  if (ng == 0) return;
+  with_harmonic(o, [&](auto RT, auto NB) {
+    k_harm_m2m<decltype(RT)::value, decltype(NB)::value><<<sy_blocks(ng * o.nb), SY_TB, 0, plan.ctx->stream>>>(
+        plan.hl[l]->sym_m2m.p, o.hN, KP, o.hchi.p, o.hrank.p, plan.parent.p, plan.has_source.p, first, ng, plan.Mp.p);
+  });
+  FFMM_LAUNCH_CHECK();
+}
+
+void sym_harmonic_l2l(Plan &plan, int l) {
+  OpCache &o = *plan.ops;
+  const int64_t ng = plan.nl[l] / NCHILD;
+  const int KP = (o.hN + SY_K - 1) / SY_K * SY_K;
+  if (ng == 0) return;
+  with_harmonic(o, [&](auto RT, auto NB) {
+    k_harm_l2l<decltype(RT)::value, decltype(NB)::value><<<sy_blocks(ng * o.nb), SY_TB, 0, plan.ctx->stream>>>(
+        plan.hl[l - 1]->sym_l2l.p, o.hN, KP, o.hchi.p, o.hrank.p, plan.parent.p, plan.lo[l], ng, plan.Pl.p);
   });
   FFMM_LAUNCH_CHECK();
 }

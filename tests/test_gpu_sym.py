@@ -56,3 +56,31 @@ def test_sources_beyond_the_lds_stage(precision):
     u = plan.matvec(tau).cpu().numpy()
     u_ref = O.FMM(cache.host_operators(), pts, 110, BOX[0], BOX[1]).matvec(tau)
     assert np.linalg.norm(u - u_ref) < (2e-6 if precision == "mixed" else 1e-11) * np.linalg.norm(u_ref)
+
+
+@pytest.mark.parametrize("kernel,p", [("laplace", 2), ("laplace", 5), ("laplace", 10), ("yukawa", 7), ("laplace", 13),
+                                      ("stokes", 3), ("stokes", 10), ("laplace", 16)])
+def test_harmonic_blocks_vs_oracle(kernel, p):
+    """M2M and L2L by reflection parity against the harmonic oracle's dense operators on the
+    same tree (1e-11, as tests/test_gpu_harmonic.py): one to three row tiles, expansions of
+    one to five chunks of 64 entries, one and four blocks, groups of 16 and of 4 columns with
+    missing ones."""
+    import ffmm
+    from test_gpu_harmonic import oracle_for
+    print(f"[sym] harmonic {kernel} p={p}", flush=True)
+    n = 1500
+    rng = np.random.default_rng(10 * p)
+    pts = rng.random((n, 3))
+    pts[: n // 3] = 0.4 + 0.05 * rng.random((n // 3, 3))
+    if kernel == "stokes":
+        m, d = ffmm.StokesHarmonics(ffmm.Stokeslet3D(), p=p), rng.standard_normal((n, 9))
+    else:
+        K = ffmm.Laplace3D() if kernel == "laplace" else ffmm.Yukawa3D(5.0)
+        m, d = ffmm.SphericalHarmonics(K, p=p), rng.standard_normal(n)
+    cache = ffmm.OperatorCache(m)
+    plan = ffmm.DevicePlan(m, pts, ppl=10, bbox=BOX, cache=cache)
+    u = plan.matvec(d).cpu().numpy()
+    tree = plan.download_tree()
+    u_ref = oracle_for(m, cache, pts, 10, tree.perm)[0].matvec(d)
+    u_ref = u_ref.reshape(u.shape)
+    assert np.max(np.abs(u - u_ref)) < 1e-11 * np.max(np.abs(u_ref))
