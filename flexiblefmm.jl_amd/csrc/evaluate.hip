@@ -3,7 +3,7 @@
 // colleagues, the target's own source excluded by index (a masked select, never a
 // multiply).
 //
-// One wavefront per real leaf, one lane per target: the surface with the leaf's local
+// One workgroup (one wavefront, or four where there are few leaves) per real leaf, one lane per target: the surface with the leaf's local
 // density, then the colleagues' sources, pass through LDS tiles that the wave loads
 // with coalesced reads and every lane then reads at the same address (a broadcast),
 // so the 64 lanes only differ in their target.  Targets at arbitrary points are
@@ -19,7 +19,6 @@
 namespace ffmm {
 
 constexpr int TB = 256;
-constexpr int EV_TB = 64;
 constexpr int EV_CK = 256;   // entries of an LDS tile: surface points with densities, or sources with charges
 constexpr double C4PI = 0.07957747154594767;   // 1 / (4 pi)
 
@@ -46,8 +45,9 @@ __device__ __forceinline__ void accumulate_masked(double d0, double d1, double d
   }
 }
 
-template <int OUT>
-__global__ void __launch_bounds__(EV_TB) k_eval(EvalArgs a) {
+template <int OUT, int EVT>
+__global__ void __launch_bounds__(EVT) k_eval(EvalArgs a) {
+  __shared__ double red[EVT > 64 ? 4 * EVT : 1];
   __shared__ double4 tile[EV_CK];
   __shared__ int32_t tile_id[EV_CK];
   __shared__ NearList nl;
@@ -67,13 +67,13 @@ __global__ void __launch_bounds__(EV_TB) k_eval(EvalArgs a) {
   const double *__restrict__ Z = a.surf + 2 * a.Nl;
   near_list(a, i, nl);
   const int32_t nsrc = nl.pre[NCOLL];
-  for (int32_t tb = t0; tb < t1; tb += EV_TB) {
-    // a tile of up to 64 targets; when it has fewer, R = 64 / ntp replicas of each
+  for (int32_t tb = t0; tb < t1; tb += EVT) {
+    // a tile of up to EVT targets; when it has fewer, R = EVT / ntp replicas of each
     // target split the surface points and the sources, and are summed at the end
-    const int cnt = min(EV_TB, t1 - tb);
+    const int cnt = min(EVT, t1 - tb);
     int ntp = 1;
     while (ntp < cnt) ntp <<= 1;
-    const int R = EV_TB / ntp;
+    const int R = EVT / ntp;
     const int tl = (int)threadIdx.x % ntp, rep = (int)threadIdx.x / ntp;
     const int32_t j = tb + tl;
     const bool valid = tl < cnt;
@@ -88,7 +88,7 @@ __global__ void __launch_bounds__(EV_TB) k_eval(EvalArgs a) {
     for (int k0 = 0; k0 < a.Nl; k0 += EV_CK) {
       const int nk = min(EV_CK, a.Nl - k0);
       __syncthreads();
-      for (int k = threadIdx.x; k < nk; k += EV_TB)
+      for (int k = threadIdx.x; k < nk; k += EVT)
         tile[k] = make_double4(X[k0 + k] * sc, Y[k0 + k] * sc, Z[k0 + k] * sc, L[k0 + k]);
       __syncthreads();
 #pragma unroll 4
@@ -103,7 +103,7 @@ __global__ void __launch_bounds__(EV_TB) k_eval(EvalArgs a) {
     for (int32_t q0 = 0; q0 < nsrc; q0 += EV_CK) {
       const int nq = min(EV_CK, nsrc - q0);
       __syncthreads();
-      for (int k = threadIdx.x; k < nq; k += EV_TB) {
+      for (int k = threadIdx.x; k < nq; k += EVT) {
         const int32_t q = near_source(nl, q0 + k);
         tile[k] = make_double4(a.sx[q], a.sy[q], a.sz[q], a.tau[q]);
         tile_id[k] = q;
@@ -115,9 +115,7 @@ __global__ void __launch_bounds__(EV_TB) k_eval(EvalArgs a) {
         accumulate_masked<OUT>(x - v.x, y - v.y, z - v.z, v.w, tile_id[k] != skip, acc);
       }
     }
-    for (int off = ntp; off < EV_TB; off <<= 1)
-#pragma unroll
-      for (int c = 0; c < 4; c++) acc[c] += __shfl_xor(acc[c], off, EV_TB);
+    sum_replicas<EVT>(acc, ntp, red);
     if (valid && rep == 0) {
       const int64_t o = self ? a.outidx[j] : a.outidx[j];
       if (OUT == FFMM_POTENTIAL) {
@@ -178,12 +176,13 @@ struct NearSrc32 {
   int32_t id;
 };
 
-template <int OUT>
-__global__ void __launch_bounds__(EV_TB) k_eval32(EvalArgs a) {
+template <int OUT, int EVT>
+__global__ void __launch_bounds__(EVT) k_eval32(EvalArgs a) {
+  __shared__ double red[EVT > 64 ? 4 * EVT : 1];
   // the potential alone: tiles of 128 entries (LDS 4.3 KB per workgroup, so more
   // workgroups per CU: 4.60 -> 4.15 ms at 4M sources); with the gradient the tiles of 256
   // measured faster
-  constexpr int CK = OUT == FFMM_POTENTIAL ? EV_CK / 2 : EV_CK;
+  constexpr int CK = OUT == FFMM_POTENTIAL && EVT == 64 ? EV_CK / 2 : EV_CK;
   __shared__ NearSrc32 tile[CK];
   __shared__ NearList nl;
   float4 *tile32 = reinterpret_cast<float4 *>(tile);
@@ -201,11 +200,11 @@ __global__ void __launch_bounds__(EV_TB) k_eval32(EvalArgs a) {
   const double *__restrict__ Z = a.surf + 2 * a.Nl;
   near_list(a, i, nl);
   const int32_t nsrc = nl.pre[NCOLL];
-  for (int32_t tb = t0; tb < t1; tb += EV_TB) {
-    const int cnt = min(EV_TB, t1 - tb);
+  for (int32_t tb = t0; tb < t1; tb += EVT) {
+    const int cnt = min(EVT, t1 - tb);
     int ntp = 1;
     while (ntp < cnt) ntp <<= 1;
-    const int R = EV_TB / ntp;
+    const int R = EVT / ntp;
     const int tl = (int)threadIdx.x % ntp, rep = (int)threadIdx.x / ntp;
     const int32_t j = tb + tl;
     const bool valid = tl < cnt;
@@ -219,7 +218,7 @@ __global__ void __launch_bounds__(EV_TB) k_eval32(EvalArgs a) {
     for (int k0 = 0; k0 < a.Nl; k0 += CK) {
       const int nk = min(CK, a.Nl - k0);
       __syncthreads();
-      for (int k = threadIdx.x; k < nk; k += EV_TB)
+      for (int k = threadIdx.x; k < nk; k += EVT)
         tile32[k] = make_float4((float)(X[k0 + k] * sc), (float)(Y[k0 + k] * sc), (float)(Z[k0 + k] * sc),
                                 (float)L[k0 + k]);
       __syncthreads();
@@ -236,7 +235,7 @@ __global__ void __launch_bounds__(EV_TB) k_eval32(EvalArgs a) {
     for (int32_t q0 = 0; q0 < nsrc; q0 += CK) {
       const int nq = min(CK, nsrc - q0);
       __syncthreads();
-      for (int k = threadIdx.x; k < nq; k += EV_TB) {
+      for (int k = threadIdx.x; k < nq; k += EVT) {
         const int32_t q = near_source(nl, q0 + k);
         tile[k] = NearSrc32{a.sx[q], a.sy[q], a.sz[q], (float)a.tau[q], q};
       }
@@ -257,9 +256,7 @@ __global__ void __launch_bounds__(EV_TB) k_eval32(EvalArgs a) {
       }
       fold32<OUT>(ks, kc, g, acc);
     }
-    for (int off = ntp; off < EV_TB; off <<= 1)
-#pragma unroll
-      for (int c = 0; c < 4; c++) acc[c] += __shfl_xor(acc[c], off, EV_TB);
+    sum_replicas<EVT>(acc, ntp, red);
     if (valid && rep == 0) {
       const int64_t o = a.outidx[j];
       if (OUT == FFMM_POTENTIAL) {
@@ -287,13 +284,18 @@ static void launch_eval(Plan &plan, EvalArgs &a, int output) {
   }
   hipStream_t s = plan.ctx->stream;
   const unsigned g = (unsigned)nleaves;
-  if (plan.precision == FFMM_PREC_MIXED) {
-    if (output == FFMM_POTENTIAL) k_eval32<FFMM_POTENTIAL><<<g, EV_TB, 0, s>>>(a);
-    else if (output == FFMM_GRADIENT) k_eval32<FFMM_GRADIENT><<<g, EV_TB, 0, s>>>(a);
-    else k_eval32<2><<<g, EV_TB, 0, s>>>(a);
-  } else if (output == FFMM_POTENTIAL) k_eval<FFMM_POTENTIAL><<<g, EV_TB, 0, s>>>(a);
-  else if (output == FFMM_GRADIENT) k_eval<FFMM_GRADIENT><<<g, EV_TB, 0, s>>>(a);
-  else k_eval<2><<<g, EV_TB, 0, s>>>(a);
+  auto go = [&](auto EVT) {
+    constexpr int n = decltype(EVT)::value;
+    if (plan.precision == FFMM_PREC_MIXED) {
+      if (output == FFMM_POTENTIAL) k_eval32<FFMM_POTENTIAL, n><<<g, n, 0, s>>>(a);
+      else if (output == FFMM_GRADIENT) k_eval32<FFMM_GRADIENT, n><<<g, n, 0, s>>>(a);
+      else k_eval32<2, n><<<g, n, 0, s>>>(a);
+    } else if (output == FFMM_POTENTIAL) k_eval<FFMM_POTENTIAL, n><<<g, n, 0, s>>>(a);
+    else if (output == FFMM_GRADIENT) k_eval<FFMM_GRADIENT, n><<<g, n, 0, s>>>(a);
+    else k_eval<2, n><<<g, n, 0, s>>>(a);
+  };
+  if (nleaves < EVAL_WIDE_LEAVES) go(std::integral_constant<int, 256>{});
+  else go(std::integral_constant<int, 64>{});
   FFMM_LAUNCH_CHECK();
 }
 

@@ -576,6 +576,39 @@ __device__ __forceinline__ void near_list(const EvalArgs &a, int i, NearList &nl
   __syncthreads();
 }
 
+// The evaluation kernels take one workgroup per leaf, of one wave or, where there are few
+// leaves, of four: with one wave each, few leaves leave the card's 1,024 SIMDs idle or with
+// too few waves to hide a tile's loads, and the largest leaves end last.  Measured, one wave
+// / four (ms):
+//   cube mixed, 20 points a leaf    9,997 leaves .109 / .079   29,037 leaves .128 / .165
+//   cube mixed, 200 points a leaf   3,676 leaves 2.19 / .84    12,937 leaves 2.90 / 1.43
+//   cube FP64, 64 points a leaf       960 leaves .241 / .091   22,149 leaves .603 / .566
+//   Stokes mixed, 64 points a leaf  1,030 leaves .486 / .172   10,130 .705 / .479   22,226 .785 / .902
+//   Yukawa mixed, 64 points a leaf    981 leaves .305 / .114    5,286 .333 / .295   10,130 .379 / .562
+// Yukawa turns first: the exponential leaves less to hide, the lanes' weights fill the LDS.
+constexpr int64_t EVAL_WIDE_LEAVES = 16384, EVAL_WIDE_LEAVES_YUKAWA = 6144;
+
+// sums of the replicas of each of ntp targets (thread t: target t % ntp) into the threads
+// below ntp; red: 4 EVT doubles (not used for one wave).  Synchronises a block of four waves.
+template <int EVT>
+__device__ __forceinline__ void sum_replicas(double acc[4], int ntp, double *red) {
+  for (int off = ntp; off < 64; off <<= 1)
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[c] += __shfl_xor(acc[c], off, 64);
+  if constexpr (EVT > 64) {
+    if (ntp == EVT) return;
+    const int t = threadIdx.x, st = ntp < 64 ? 64 : ntp;
+#pragma unroll
+    for (int c = 0; c < 4; c++) red[c * EVT + t] = acc[c];
+    __syncthreads();
+    if (t < ntp)
+      for (int r = st; r < EVT; r += st)
+#pragma unroll
+        for (int c = 0; c < 4; c++) acc[c] += red[c * EVT + t + r];
+    __syncthreads();
+  }
+}
+
 // the source index of entry f of the list (0 <= f < pre[NCOLL]): the last m with pre[m] <= f
 __device__ __forceinline__ int32_t near_source(const NearList &nl, int32_t f) {
   int m = 0, h = NCOLL;

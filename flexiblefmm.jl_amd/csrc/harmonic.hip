@@ -530,9 +530,10 @@ __device__ __forceinline__ HTab32 eval_tables<float>(const EvalArgs &a) { return
 // near field's FP32 partial sums are folded into FP64 accumulators after every LDS tile
 // (the FP32 evaluation of the mixed form, src/device.jl:186-206 with Float32 locals and
 // densities).
-template <class T, int KIND, int OUT>
-__global__ void __launch_bounds__(HB) k_eval_harm(EvalArgs a) {
+template <class T, int KIND, int OUT, int EVT>
+__global__ void __launch_bounds__(EVT) k_eval_harm(EvalArgs a) {
   extern __shared__ double sm[];
+  __shared__ double red[EVT > 64 ? 4 * EVT : 1];
   constexpr bool F32 = sizeof(T) == 4;
   // FP64: doubles per tile entry, position and density components (Stokes 9, Laplace a
   // charge and a dipole, Yukawa a charge); FP32: an HNearSrc32 with ND densities
@@ -553,9 +554,9 @@ __global__ void __launch_bounds__(HB) k_eval_harm(EvalArgs a) {
   const HTabT<T> tb = eval_tables<T>(a);
   T *L = reinterpret_cast<T *>(sm);                   // the leaf's local expansion
   double *uw = sm + (NB * sizeof(T) + 7) / 8;         // per lane: radial weights to p (Yukawa potential)
-  double *ug = uw + HB * (p + 2);                     // per lane: radial weights to p + 1 (Yukawa gradient)
+  double *ug = uw + EVT * (p + 2);                     // per lane: radial weights to p + 1 (Yukawa gradient)
   const double *Lg = a.Lc + (int64_t)s * NB;
-  for (int k = threadIdx.x; k < NB; k += HB) L[k] = (T)Lg[k];
+  for (int k = threadIdx.x; k < NB; k += EVT) L[k] = (T)Lg[k];
   __syncthreads();
   const double c0 = a.centers[i], c1 = a.centers[a.nn + i], c2 = a.centers[2 * a.nn + i];
   const int lv = a.level[i];
@@ -565,11 +566,11 @@ __global__ void __launch_bounds__(HB) k_eval_harm(EvalArgs a) {
   __shared__ int32_t tile_id[HT_CK];
   near_list(a, i, nl);
   const int32_t nsrc = nl.pre[NCOLL];
-  for (int32_t tbk = t0; tbk < t1; tbk += HB) {
-    const int cnt = min(HB, t1 - tbk);
+  for (int32_t tbk = t0; tbk < t1; tbk += EVT) {
+    const int cnt = min(EVT, t1 - tbk);
     int ntp = 1;
     while (ntp < cnt) ntp <<= 1;
-    const int R = HB / ntp;
+    const int R = EVT / ntp;
     const int tl = (int)threadIdx.x % ntp, rep = (int)threadIdx.x / ntp;
     const int32_t j = tbk + tl;
     const bool valid = tl < cnt;
@@ -687,7 +688,7 @@ __global__ void __launch_bounds__(HB) k_eval_harm(EvalArgs a) {
       for (int32_t q0 = 0; q0 < nsrc; q0 += HT_CK) {
         const int nq = min(HT_CK, nsrc - q0);
         __syncthreads();
-        for (int k = threadIdx.x; k < nq; k += HB) {
+        for (int k = threadIdx.x; k < nq; k += EVT) {
           const int32_t q = near_source(nl, q0 + k);
           double *e = tile + k * TW;
           e[0] = a.sx[q];
@@ -708,7 +709,7 @@ __global__ void __launch_bounds__(HB) k_eval_harm(EvalArgs a) {
       for (int32_t q0 = 0; q0 < nsrc; q0 += HT_CK32) {
         const int nq = min(HT_CK32, nsrc - q0);
         __syncthreads();
-        for (int k = threadIdx.x; k < nq; k += HB) tile32[k] = near_src32<KIND>(a, near_source(nl, q0 + k));
+        for (int k = threadIdx.x; k < nq; k += EVT) tile32[k] = near_src32<KIND>(a, near_source(nl, q0 + k));
         __syncthreads();
         for (int k = rep; k < nq; k += R) {
           const HNearSrc32<KIND> e = tile32[k];
@@ -721,9 +722,7 @@ __global__ void __launch_bounds__(HB) k_eval_harm(EvalArgs a) {
         }
       }
     }
-    for (int off = ntp; off < HB; off <<= 1)
-#pragma unroll
-      for (int c = 0; c < 4; c++) acc[c] += __shfl_xor(acc[c], off, HB);
+    sum_replicas<EVT>(acc, ntp, red);
     if (valid && rep == 0) {
       const int64_t o = a.outidx[j];
       if (KIND == 2 && OUT == FFMM_PRESSURE) {
@@ -771,32 +770,43 @@ void harmonic_s2m_level(Plan &plan, int l) {
   FFMM_LAUNCH_CHECK();
 }
 
-template <class T>
-static void launch_eval_harm(const OpCache &o, const EvalArgs &a, int output, unsigned g, hipStream_t s) {
-  const size_t lds = ((size_t)o.Ns * sizeof(T) + 7) / 8 * 8 +
-                     (o.kernel == FFMM_KERNEL_YUKAWA ? 2 * sizeof(double) * HB * (o.p + 2) : 0);
+template <class T, int EVT>
+static void launch_eval_harm(const OpCache &o, const EvalArgs &a, int output, unsigned g, size_t lds, hipStream_t s) {
   if (o.kernel == FFMM_KERNEL_STOKESLET) {
-    if (output == FFMM_PRESSURE) k_eval_harm<T, 2, FFMM_PRESSURE><<<g, HB, lds, s>>>(a);
-    else k_eval_harm<T, 2, FFMM_POTENTIAL><<<g, HB, lds, s>>>(a);
+    if (output == FFMM_PRESSURE) k_eval_harm<T, 2, FFMM_PRESSURE, EVT><<<g, EVT, lds, s>>>(a);
+    else k_eval_harm<T, 2, FFMM_POTENTIAL, EVT><<<g, EVT, lds, s>>>(a);
   } else if (o.kernel == FFMM_KERNEL_LAPLACE) {
-    if (output == FFMM_POTENTIAL) k_eval_harm<T, 0, FFMM_POTENTIAL><<<g, HB, lds, s>>>(a);
-    else if (output == FFMM_GRADIENT) k_eval_harm<T, 0, FFMM_GRADIENT><<<g, HB, lds, s>>>(a);
-    else k_eval_harm<T, 0, FFMM_POTENTIAL_GRADIENT><<<g, HB, lds, s>>>(a);
+    if (output == FFMM_POTENTIAL) k_eval_harm<T, 0, FFMM_POTENTIAL, EVT><<<g, EVT, lds, s>>>(a);
+    else if (output == FFMM_GRADIENT) k_eval_harm<T, 0, FFMM_GRADIENT, EVT><<<g, EVT, lds, s>>>(a);
+    else k_eval_harm<T, 0, FFMM_POTENTIAL_GRADIENT, EVT><<<g, EVT, lds, s>>>(a);
   } else {
-    if (output == FFMM_POTENTIAL) k_eval_harm<T, 1, FFMM_POTENTIAL><<<g, HB, lds, s>>>(a);
-    else if (output == FFMM_GRADIENT) k_eval_harm<T, 1, FFMM_GRADIENT><<<g, HB, lds, s>>>(a);
-    else k_eval_harm<T, 1, FFMM_POTENTIAL_GRADIENT><<<g, HB, lds, s>>>(a);
+    if (output == FFMM_POTENTIAL) k_eval_harm<T, 1, FFMM_POTENTIAL, EVT><<<g, EVT, lds, s>>>(a);
+    else if (output == FFMM_GRADIENT) k_eval_harm<T, 1, FFMM_GRADIENT, EVT><<<g, EVT, lds, s>>>(a);
+    else k_eval_harm<T, 1, FFMM_POTENTIAL_GRADIENT, EVT><<<g, EVT, lds, s>>>(a);
   }
   FFMM_LAUNCH_CHECK();
+}
+template <class T>
+static void launch_eval_harm(const OpCache &o, const EvalArgs &a, int output, int64_t nleaves, hipStream_t s) {
+  // per workgroup: the leaf's expansion and, Yukawa, each lane's radial weights
+  auto lds = [&](int evt) {
+    return ((size_t)o.Ns * sizeof(T) + 7) / 8 * 8 +
+           (o.kernel == FFMM_KERNEL_YUKAWA ? 2 * sizeof(double) * evt * (o.p + 2) : 0);
+  };
+  // four waves where there are few leaves, unless the weights of 256 lanes (p > 12) fill the LDS
+  const int64_t wide = o.kernel == FFMM_KERNEL_YUKAWA ? EVAL_WIDE_LEAVES_YUKAWA : EVAL_WIDE_LEAVES;
+  if (nleaves < wide && lds(256) <= 64 * 1024)
+    launch_eval_harm<T, 256>(o, a, output, (unsigned)nleaves, lds(256), s);
+  else
+    launch_eval_harm<T, 64>(o, a, output, (unsigned)nleaves, lds(64), s);
 }
 
 // the mixed form evaluates in FP32 (k_eval_harm<float>), the FP64 form in FP64
 void launch_eval_harmonic(Plan &plan, const EvalArgs &a, int output) {
   const int64_t nleaves = plan.leaf_off[plan.L];
   if (nleaves == 0) return;
-  const unsigned g = (unsigned)nleaves;
-  if (plan.precision == FFMM_PREC_MIXED) launch_eval_harm<float>(*plan.ops, a, output, g, plan.ctx->stream);
-  else launch_eval_harm<double>(*plan.ops, a, output, g, plan.ctx->stream);
+  if (plan.precision == FFMM_PREC_MIXED) launch_eval_harm<float>(*plan.ops, a, output, nleaves, plan.ctx->stream);
+  else launch_eval_harm<double>(*plan.ops, a, output, nleaves, plan.ctx->stream);
 }
 
 }  // namespace ffmm
