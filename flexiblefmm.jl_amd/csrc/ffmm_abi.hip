@@ -367,7 +367,19 @@ static void upload_signed_tables(OpCache &o, const int32_t *idx, const int8_t *s
     }
   o.gsel.upload(g.data(), n, s);
   o.ssel.upload(t.data(), n, s);
-  o.fsel.upload(fw.data(), n, s);
+  std::vector<uint8_t> g8, f8;
+  if (N <= FM_MAXN) {
+    g8.assign((size_t)NFAR * 128, 0);
+    f8.assign((size_t)NFAR * 128, FM_MAXN);
+    for (int f = 0; f < NFAR; f++)
+      for (int i = 0; i < N; i++) {
+        const int32_t a = g[(size_t)f * N + i], b = fw[(size_t)f * N + i];
+        g8[(size_t)f * 128 + i] = (uint8_t)((a & 0x7f) | (a < 0 ? 0x80 : 0));
+        f8[(size_t)f * 128 + i] = (uint8_t)((b & 0x7f) | (b < 0 ? 0x80 : 0));
+      }
+    o.gsel8.upload(g8.data(), g8.size(), s);
+    o.fsel8.upload(f8.data(), f8.size(), s);
+  }
   FFMM_HIP(hipStreamSynchronize(s));   // before the host tables go
 }
 
@@ -676,13 +688,33 @@ int ffmm_opcache_put_harmonic_level(ffmm_opcache cache, double width, const doub
     lv->reps.upload(reps, (size_t)o.nclass * N * N, s);
     std::vector<float> r32(reps, reps + (size_t)o.nclass * N * N);   // the mixed form's class GEMMs
     lv->reps32.upload(r32.data(), r32.size(), s);
-    std::vector<float> rr;   // held until the copies are done
-    if (N <= 128) {
-      rr.assign((size_t)o.nclass * 128 * 128, 0.f);
+    std::vector<uint16_t> rb;   // held until the copies are done
+    if (N <= FM_MAXN) {
+      auto bf16 = [](double x) {   // round to nearest even
+        const float f = (float)x;
+        uint32_t u;
+        memcpy(&u, &f, 4);
+        return (uint16_t)((u + 0x7fff + ((u >> 16) & 1)) >> 16);
+      };
+      auto value = [](uint16_t b) {
+        const uint32_t u = (uint32_t)b << 16;
+        float f;
+        memcpy(&f, &u, 4);
+        return (double)f;
+      };
+      rb.assign((size_t)o.nclass * 128 * 128 * 3, 0);
       for (int c = 0; c < o.nclass; c++)
         for (int k = 0; k < N; k++)
-          for (int i = 0; i < N; i++) rr[((size_t)c * 128 + i) * 128 + k] = r32[(size_t)c * N * N + i + (size_t)N * k];
-      lv->reps32r.upload(rr.data(), rr.size(), s);
+          for (int i = 0; i < N; i++) {
+            // row 16 w + li, k = 32 kb + 8 lk + j
+            const size_t at = (((((size_t)c * 8 + i / 16) * 4 + k / 32) * 3) * 64 + (k / 8 % 4) * 16 + i % 16) * 8 + k % 8;
+            double x = r32[(size_t)c * N * N + i + (size_t)N * k];
+            for (int q = 0; q < 3; q++) {
+              rb[at + (size_t)q * 64 * 8] = bf16(x);
+              x -= value(rb[at + (size_t)q * 64 * 8]);
+            }
+          }
+      lv->repsb.upload(rb.data(), rb.size(), s);
     }
     ctx.sync();
     std::lock_guard<std::mutex> lk(o.hmu);

@@ -216,6 +216,8 @@ struct Context {
 constexpr int METHOD_CUBE = 0;       // CubeKernelIndependent{3}(Laplace3D())
 constexpr int METHOD_HARMONIC = 1;   // SphericalHarmonics (Laplace3D, Yukawa3D), StokesHarmonics
 
+constexpr int FM_MAXN = 123;   // the fused mixed M2L: coefficients per block, N <= FM_MAXN
+
 // the operators of the harmonic methods for boxes of one width
 struct HarmonicLevel {
   double w = 0.0;
@@ -225,7 +227,10 @@ struct HarmonicLevel {
   DBuf<double> M2M, L2L;
   DBuf<double> reps;       // nclass x (N x N)
   DBuf<float> reps32;      // the same in FP32 (the mixed form's M2L)
-  DBuf<float> reps32r;     // FP32, row-major, zero-padded to 128 x 128 per class (N <= 128: the fused mixed M2L)
+  // N <= FM_MAXN, the fused mixed M2L: each FP32 entry as three bfloat16 pieces, zero-padded
+  // to 128 x 128 per class, in the order the matrix instructions read them:
+  // [class][row tile 16][K block 32][piece][lane][8]
+  DBuf<uint16_t> repsb;
 };
 
 // device pointers of the recurrence tables (HarmonicTables, src/operators/harmonics.jl:163-187)
@@ -295,8 +300,10 @@ struct OpCache {
   // the same permutations with their signs in the top bit: gsel[f, i] = idx[f, i] (sign
   // sgn[f, i]); ssel[f, j] = i = inv[f, j] (sign sgn_t[f, i]); one load per entry
   DBuf<int32_t> gsel, ssel;
-  // fsel[f, i] = the target-frame position j of product entry i (inv[f, j] = i), sign sgn_t[f, i]
-  DBuf<int32_t> fsel;
+  // N <= FM_MAXN, a byte per entry (index, sign in the top bit), rows of 128: gsel8 as gsel;
+  // fsel8[f, i] = the target-frame position j of product entry i (inv[f, j] = i), sign sgn_t[f, i]
+  // (the padding of fsel8 points at FM_MAXN, which no column holds)
+  DBuf<uint8_t> gsel8, fsel8;
   DBuf<int8_t> sgn;
   // the spectral M2L's table operands (spectral.hip: k_had_fragments), bfloat16 and FP64
   DBuf<uint16_t> had_mixed;
@@ -574,6 +581,17 @@ __device__ __forceinline__ void near_list(const EvalArgs &a, int i, NearList &nl
   }
   if (t == 0) nl.pre[0] = 0;
   __syncthreads();
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_bf16(f32x2 v) {   // round to nearest even, both at once
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+__device__ __forceinline__ f32x2 unpack_bf16(uint32_t b) {
+  return f32x2{__uint_as_float(b << 16), __uint_as_float(b & 0xffff0000u)};
 }
 
 // The evaluation kernels take one workgroup per leaf, of one wave or, where there are few

@@ -312,140 +312,252 @@ __global__ void k_chunk_gather(T *__restrict__ Gc, const double *__restrict__ Mp
   }
 }
 
-typedef float fm_f32x4 __attribute__((ext_vector_type(4)));
 constexpr int FM_TB = 512;      // 8 waves: wave w holds the operator's row tile w (rows 16 w .. 16 w + 15)
-constexpr int FM_COLS = 128;    // product columns per tile: 8 column tiles of 16
-constexpr int FM_MP = 128;      // operator rows and K, padded: N <= 128
-constexpr int FM_BS = 132;      // LDS stride of a gathered column (16-byte aligned, K contiguous)
+constexpr int FM_COLS = 64;     // product columns per tile: 4 column tiles of 16
+constexpr int FM_BS = FM_MAXN + 1;   // LDS stride of a product column, the last entry for the rows beyond N
+
+// entry i of a wave-uniform array: the address as a scalar base and a 32-bit offset
+template <class T>
+__device__ __forceinline__ T at32(const T *base, uint32_t i) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + i * (uint32_t)sizeof(T));
+}
 
 // The class M2L of the harmonic methods in the mixed form, fused: for each tile of a
 // class's pairs in the chunk, the gathered source expansions (P_f^T m per block, signed,
 // the Stokes coupling folded into the fourth block, src/device_passes.jl:449-473) go
-// straight into LDS as FP32 and are multiplied by the class operator on FP32 MFMA
-// (v_mfma_f32_16x16x4f32).  Each wave loads its 16 operator rows per tile from a
-// row-major copy of the class operators padded to 128 x 128 (L2-resident), while the
-// other waves finish the gather, so that no register is held across the tile's phases;
-// the four K slots of an MFMA step take four consecutive k, so a lane's operands for
-// 16 k come in one 16-byte load, of the operator and of the gathered column alike.  The
-// products are written in each pair's target frame (entry j = fsel position, sign
-// applied), so the scatter adds contiguous columns.  N = (p + 1)^2 <= 128.
-template <int NB>
-__global__ void __launch_bounds__(FM_TB) __attribute__((amdgpu_waves_per_eu(4))) k_class_m2l32(float *__restrict__ Yc, const double *__restrict__ Mp,
-                                                          int Ns, int N, const float *__restrict__ reps32r,
-                                                          const int32_t *__restrict__ csrc,
-                                                          const int32_t *__restrict__ cfar,
-                                                          const int32_t *__restrict__ gsel,
-                                                          const int32_t *__restrict__ fsel,
-                                                          const double *__restrict__ offs, ChunkArgs ca,
-                                                          int32_t ntiles, const int32_t *__restrict__ ctgt) {
+// straight into LDS and are multiplied by the class operator.  The products are staged in
+// each pair's target frame (entry j = fsel position, sign applied), so the scatter adds
+// contiguous columns.  N = (p + 1)^2 <= FM_MAXN.
+//
+// Each FP32 operand is three bfloat16 pieces (the whole FP32 mantissa), the products of
+// pieces down to 2^-24 on v_mfma_f32_16x16x32_bf16 with the small ones in accumulators of
+// their own: 96 cycles per 16 x 16 block of 32 K where v_mfma_f32_16x16x4_f32 takes 256.
+// The form before (FP32 matrix instructions) gathered, multiplied and staged each tile in
+// turn behind five barriers.  Here a wave keeps its operator rows while the class lasts, and
+// the loads of a tile are in flight during the one before it (the pairs three tiles ahead,
+// their permutation bytes one); half of a tile's expansions are loaded behind the products,
+// because all of them beside the operator's 48 registers spill.  Loads return in order: a
+// tile's own go before the next tile's, or waiting for them waits for all.  Products and
+// gathered columns have LDS of their own (two workgroups per CU fill its 160 KB), so that
+// two barriers a tile are left.  A column's 16-byte chunks are stored at chunk ^ column:
+// reads and writes touch each bank once.  Measured: 1M Stokes points, p = 10, 16.3 -> 8.5 ms
+// (10.5 with spilled registers and waits in the wrong order), 200k Yukawa points 3.5 -> 1.9
+// with the scatter.  At the larger one the matrix cores are busy 36% of the time and LDS 41%,
+// 11.5 GB are fetched and 6.9 GB written beyond the L2 (2.3 TB/s): what is left is latency
+// between the two barriers.
+// KB: K blocks of 32, ceil(N / 32)
+template <int NB, int KB>
+__global__ void __launch_bounds__(FM_TB) __attribute__((amdgpu_waves_per_eu(4)))
+k_class_m2l32(float *__restrict__ Yc, const double *__restrict__ Mp, int Ns, int N, const bf16x8 *__restrict__ ops,
+              const int32_t *__restrict__ csrc, const int32_t *__restrict__ cfar, const uint32_t *__restrict__ gsel8,
+              const uint32_t *__restrict__ fsel8, const double *__restrict__ offs, ChunkArgs ca, int32_t ntiles,
+              const int32_t *__restrict__ ctgt) {
   constexpr int PPT = FM_COLS / NB;   // pairs per tile
-  __shared__ float Bs[FM_COLS * FM_BS];
-  __shared__ int32_t pf[PPT], ps[PPT], pt[PPT];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  constexpr int PW = PPT / 8;         // pairs a wave gathers
+  constexpr int PLANE = FM_COLS * 64; // words of a plane of pieces: 128 k of each column
+  __shared__ __attribute__((aligned(16))) uint32_t Bp[3 * PLANE];
+  __shared__ float Ys[FM_COLS * FM_BS];
+  __shared__ int32_t pf[2][PPT], pt[2][PPT];   // offsets and targets of a tile's pairs, by its parity
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lk = lane >> 4;
-  const int nkb = (N + 15) >> 4;      // K blocks of 16
   const bool rows = 16 * w < N;       // this wave's row tile holds operator rows
   const int32_t t0 = (int32_t)((int64_t)blockIdx.x * ntiles / gridDim.x);
   const int32_t t1 = (int32_t)((int64_t)(blockIdx.x + 1) * ntiles / gridDim.x);
-  // the K padding of the gathered columns: zero (the gather and the staging write k < N only)
-  const int kpad = 16 * nkb - N;
-  for (int e = tid; e < FM_COLS * kpad; e += FM_TB) Bs[(e / kpad) * FM_BS + N + e % kpad] = 0.f;
-  for (int32_t tile = t0; tile < t1; tile++) {
+  struct Tile {
+    int32_t c, p0, q0, npt;           // class, first pair, first chunk column, pairs
+  };
+  auto next_tile = [&](Tile &t, int32_t tile) {   // tile >= the one t held; the last one again past the end
+    tile = min(tile, t1 - 1);
+    int c = t.c;
+    while (ca.to[c + 1] <= tile) c++;
+    const int32_t lp0 = (tile - ca.to[c]) * PPT;
+    t.c = c;
+    t.p0 = ca.cs[c] + lp0;
+    t.q0 = ca.co[c] + lp0;
+    t.npt = min(PPT, ca.co[c + 1] - t.q0);
+  };
+  int32_t f0[PW], f1[PW], s1[PW], f2[PW], s2[PW];
+  uint32_t gw[PW], sg, sn = 0;        // permutation words of the next tile; signs of this one and of the next
+  double m[PW][2][NB];
+  auto load_pairs = [&](const Tile &t, int32_t *f, int32_t *s) {
+#pragma unroll
+    for (int e = 0; e < PW; e++) {
+      const int32_t p = t.p0 + min(w * PW + e, t.npt - 1);
+      f[e] = cfar[p];
+      s[e] = csrc[p];
+    }
+  };
+  auto load_words = [&](const int32_t *f) {   // entries 2 lane, 2 lane + 1 are half of a word
+#pragma unroll
+    for (int e = 0; e < PW; e++) gw[e] = at32<uint32_t>(gsel8 + f[e] * 32, lane >> 1);
+  };
+  auto load_m = [&](const int32_t *s, int e0, int e1) {
+#pragma unroll
+    for (int e = e0; e < e1; e++) {
+      const uint32_t h = gw[e] >> (16 * (lane & 1));
+      const double *__restrict__ x = Mp + (int64_t)s[e] * Ns;
+      sn |= ((h >> 7) & 1) << (2 * e) | ((h >> 15) & 1) << (2 * e + 1);
+#pragma unroll
+      for (int b = 0; b < NB; b++) {
+        m[e][0][b] = at32<double>(x + b * N, h & 127);
+        m[e][1][b] = at32<double>(x + b * N, (h >> 8) & 127);
+      }
+    }
+  };
+  // the pairs' columns as pieces: lane k / 2 holds entries k and k + 1, zero beyond N
+  auto store_columns = [&]() {
+    const bool k0 = 2 * lane < N, k1 = 2 * lane + 1 < N;
+#pragma unroll
+    for (int e = 0; e < PW; e++) {
+      if (NB == 4) {
+        const double ox = offs[3 * f0[e]], oy = offs[3 * f0[e] + 1], oz = offs[3 * f0[e] + 2];
+#pragma unroll
+        for (int z = 0; z < 2; z++)
+          m[e][z][NB - 1] += ox * m[e][z][0] + oy * m[e][z][1 % NB] + oz * m[e][z][2 % NB];
+      }
+      const uint32_t g0 = (sg >> (2 * e)) << 31, g1 = (sg >> (2 * e + 1)) << 31;
+#pragma unroll
+      for (int b = 0; b < NB; b++) {
+        const float a0 = __uint_as_float(__float_as_uint((float)m[e][0][b]) ^ g0);
+        const float a1 = __uint_as_float(__float_as_uint((float)m[e][1][b]) ^ g1);
+        const f32x2 v = f32x2{k0 ? a0 : 0.f, k1 ? a1 : 0.f};
+        const uint32_t h0 = pack_bf16(v);
+        const f32x2 r1 = v - unpack_bf16(h0);
+        const uint32_t h1 = pack_bf16(r1);
+        const uint32_t h2 = pack_bf16(r1 - unpack_bf16(h1));
+        const int col = (w * PW + e) * NB + b;
+        uint32_t *__restrict__ o = Bp + col * 64 + (((lane >> 2) ^ (col & 15)) << 2) + (lane & 3);
+        o[0] = h0;
+        o[PLANE] = h1;
+        o[2 * PLANE] = h2;
+      }
+    }
+  };
+  Tile T0, T1, T3;
+  {
     int c = 0, h = ca.nclass;
     while (h - c > 1) {
-      const int m = (c + h) >> 1;
-      if (ca.to[m] <= tile) c = m;
-      else h = m;
+      const int mid = (c + h) >> 1;
+      if (ca.to[mid] <= t0) c = mid;
+      else h = mid;
     }
-    const int32_t lp0 = (tile - ca.to[c]) * PPT;                       // first class-local pair
-    const int npt = min(PPT, ca.co[c + 1] - ca.co[c] - lp0);           // pairs in the tile
-    if (tid < npt) {
-      const int32_t p = ca.cs[c] + lp0 + tid;
-      pf[tid] = cfar[p];
-      ps[tid] = csrc[p];
-      pt[tid] = ctgt[p];
+    T0.c = c;
+  }
+  next_tile(T0, t0);
+  T1 = T0;
+  next_tile(T1, t0 + 1);
+  T3 = T1;
+  next_tile(T3, t0 + 2);
+  load_pairs(T0, f0, s1);
+  load_words(f0);
+  load_m(s1, 0, PW);
+  sg = sn;
+  load_pairs(T1, f1, s1);
+  load_words(f1);
+  load_pairs(T3, f2, s2);
+  Tile T2 = T3;
+  int32_t nf, nt;
+  if (tid < PPT) {
+    pf[0][tid] = cfar[T0.p0 + min(tid, T0.npt - 1)];
+    pt[0][tid] = ctgt[T0.p0 + min(tid, T0.npt - 1)];
+  }
+  nf = cfar[T1.p0 + min(tid, T1.npt - 1)];
+  nt = ctgt[T1.p0 + min(tid, T1.npt - 1)];
+  lds_barrier();
+  bf16x8 A[KB][3];
+  int32_t cur = -1;
+  for (int32_t tile = t0; tile < t1; tile++) {
+    const int par = (tile - t0) & 1;
+    const int32_t *__restrict__ ptb = pt[par];
+    store_columns();
+    // loads return in order: what this tile still needs goes before the next tile's loads
+    if (rows && T0.c != cur) {
+      cur = T0.c;
+      const bf16x8 *__restrict__ Ar = ops + ((size_t)cur * 8 + w) * (4 * 3 * 64) + lane;
+#pragma unroll
+      for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+        for (int q = 0; q < 3; q++) A[kb][q] = Ar[(kb * 3 + q) * 64];
+      __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0) here, so that no wait is left for the tiles that skip this
     }
-    __syncthreads();
-    // gather: a wave per pair, a lane per coefficient, all blocks
-    for (int pl = w; pl < npt; pl += FM_TB / 64)
-      for (int k = lane; k < N; k += 64) {
-        const int32_t f = pf[pl];
-        const int32_t g = gsel[f * N + k];
-        const double *__restrict__ m = Mp + (int64_t)ps[pl] * Ns + (g & 0x7fffffff);
-        const double sg = g < 0 ? -1.0 : 1.0;
-        if (NB == 4) {
-          const double m0 = m[0], m1 = m[N], m2 = m[2 * N], m3 = m[3 * N];
-          float *__restrict__ b = Bs + (pl * 4) * FM_BS + k;
-          b[0] = (float)(sg * m0);
-          b[FM_BS] = (float)(sg * m1);
-          b[2 * FM_BS] = (float)(sg * m2);
-          b[3 * FM_BS] = (float)(sg * (m3 + offs[3 * f] * m0 + offs[3 * f + 1] * m1 + offs[3 * f + 2] * m2));
-        } else {
-          Bs[pl * FM_BS + k] = (float)(sg * m[0]);
-        }
-      }
-    // operator row 16 w + li, k = 16 kb + 4 lk + q (q < 4): one 16-byte load per kb from
-    // the padded row-major table (zero beyond N), in flight while the other waves gather
-    fm_f32x4 a4[8];
+    uint32_t fw[FM_COLS / 16];
+#pragma unroll
+    for (int ct = 0; ct < FM_COLS / 16; ct++) fw[ct] = at32<uint32_t>(fsel8, pf[par][ct * (16 / NB) + li / NB] * 32 + 4 * w + lk);
+    // the next tile's expansions: half here, half behind the products (all at once spills)
+    sn = 0;
+    load_m(s1, 0, PW / 2);
+    next_tile(T3, tile + 3);
+    int32_t f3[PW], s3[PW];
+    load_pairs(T3, f3, s3);
+    lds_barrier();
+    if (tid < PPT) {   // the next tile's: every wave is past the tile before this one
+      pf[par ^ 1][tid] = nf;
+      pt[par ^ 1][tid] = nt;
+    }
+    {
+      nf = at32<int32_t>(cfar + T2.p0, min(tid, T2.npt - 1));
+      nt = at32<int32_t>(ctgt + T2.p0, min(tid, T2.npt - 1));
+    }
     if (rows) {
-      const float *__restrict__ Ar = reps32r + ((size_t)c * FM_MP + 16 * w + li) * FM_MP + 4 * lk;
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int kb = 0; kb < 8; kb++) a4[kb] = *reinterpret_cast<const fm_f32x4 *>(Ar + 16 * kb);
-    }
-    __syncthreads();
-    // products: wave w, row tile w, all 8 column tiles
-    fm_f32x4 acc[8];
+      for (int ct = 0; ct < FM_COLS / 16; ct++) {
+        f32x4 c0 = f32x4{0.f, 0.f, 0.f, 0.f}, c1 = c0, c2 = c0;
 #pragma unroll
-    for (int ct = 0; ct < 8; ct++) acc[ct] = fm_f32x4{0.f, 0.f, 0.f, 0.f};
-    if (rows) {
-      const float *__restrict__ bb = Bs + li * FM_BS + 4 * lk;
-#pragma unroll
-      for (int kb = 0; kb < 8; kb++) {
-        if (kb < nkb) {
-#pragma unroll
-          for (int ct = 0; ct < 8; ct++) {
-            const fm_f32x4 b4 = *reinterpret_cast<const fm_f32x4 *>(bb + 16 * ct * FM_BS + 16 * kb);
-#pragma unroll
-            for (int q = 0; q < 4; q++) acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[kb][q], b4[q], acc[ct], 0, 0, 0);
-          }
+        for (int kb = 0; kb < KB; kb++) {
+          const uint32_t *p = Bp + (16 * ct + li) * 64 + (((4 * kb + lk) ^ li) << 2);
+          const bf16x8 b0 = *reinterpret_cast<const bf16x8 *>(p);
+          const bf16x8 b1 = *reinterpret_cast<const bf16x8 *>(p + PLANE);
+          const bf16x8 b2 = *reinterpret_cast<const bf16x8 *>(p + 2 * PLANE);
+          c0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[kb][0], b0, c0, 0, 0, 0);
+          c1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[kb][1], b0, c1, 0, 0, 0);
+          c2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[kb][2], b0, c2, 0, 0, 0);
+          c1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[kb][0], b1, c1, 0, 0, 0);
+          c2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[kb][1], b1, c2, 0, 0, 0);
+          c2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[kb][0], b2, c2, 0, 0, 0);
         }
+        // lane (lk, li) holds rows 16 w + 4 lk + r of column 16 ct + li
+        const f32x4 v = c0 + (c1 + c2);
+        float *__restrict__ y = Ys + (16 * ct + li) * FM_BS;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const uint32_t h = fw[ct] >> (8 * r);
+          y[h & 127] = __uint_as_float(__float_as_uint(v[r]) ^ ((h & 128) << 24));
+        }
+        __builtin_amdgcn_sched_barrier(0);   // a column tile at a time: the registers of one
       }
     }
-    __syncthreads();   // every wave's reads of Bs are done: Bs becomes the staging of the products
-    if (rows) {
-#pragma unroll
-      for (int ct = 0; ct < 8; ct++) {
-        const int col = 16 * ct + li, pl = col / NB;
-        if (pl < npt) {
-          const int32_t f = pf[pl];
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const int i = 16 * w + 4 * lk + r;
-            if (i < N) {
-              const int32_t fs = fsel[f * N + i];
-              Bs[col * FM_BS + (fs & 0x7fffffff)] = fs < 0 ? -acc[ct][r] : acc[ct][r];
-            }
-          }
-        }
-      }
-    }
-    __syncthreads();
-    // coalesced copy of the tile's columns (pair column q = co[c] + lp0 + pl, NB N
-    // entries), the products of consecutive pairs of one target summed first: the first
-    // pair of each such run carries the run's sum, the others are not written
-    float *__restrict__ out = Yc + ((int64_t)ca.co[c] + lp0) * NB * N;
-    for (int col = w; col < npt * NB; col += FM_TB / 64) {
+    load_m(s1, PW / 2, PW);
+    sg = sn;
+    load_words(f2);
+    lds_barrier();   // the products are staged, and every read of the gathered columns is done
+    // coalesced copy of the tile's columns (pair column q0 + pl, NB N entries), the products
+    // of consecutive pairs of one target summed first: the first pair of each such run
+    // carries the run's sum, the others are not written
+    float *__restrict__ out = Yc + (int64_t)T0.q0 * NB * N;
+    for (int col = w; col < T0.npt * NB; col += FM_TB / 64) {
       const int pl = col / NB, b = col - pl * NB;
-      if (pl > 0 && pt[pl] == pt[pl - 1]) continue;
+      const int32_t tg = ptb[pl];
+      if (pl > 0 && tg == ptb[pl - 1]) continue;
       int pe = pl + 1;
-      while (pe < npt && pt[pe] == pt[pl]) pe++;
+      while (pe < T0.npt && ptb[pe] == tg) pe++;
       for (int j = lane; j < N; j += 64) {
-        float acc = Bs[col * FM_BS + j];
-        for (int r = pl + 1; r < pe; r++) acc += Bs[(r * NB + b) * FM_BS + j];
+        float acc = Ys[col * FM_BS + j];
+        for (int r = pl + 1; r < pe; r++) acc += Ys[(r * NB + b) * FM_BS + j];
         out[(int64_t)col * N + j] = acc;
       }
     }
-    __syncthreads();   // before the next tile's pair list and gather (the K padding is never written)
+    T0 = T1;
+    T1 = T2;
+    T2 = T3;
+#pragma unroll
+    for (int e = 0; e < PW; e++) {
+      f0[e] = f1[e];
+      f1[e] = f2[e];
+      s1[e] = s2[e];
+      f2[e] = f3[e];
+      s2[e] = s3[e];
+    }
   }
 }
 
@@ -626,10 +738,10 @@ static void gemm32(Context &ctx, int m, int n, int k, const float *A, int lda, c
                           C, ldc));
 }
 
-// the harmonic methods in the mixed form with at most 128 coefficients per block take
+// the harmonic methods in the mixed form with at most FM_MAXN coefficients per block take
 // the fused gather + product kernel
 static bool fused_m2l(const OpCache &o) {
-  return o.method == METHOD_HARMONIC && o.hN <= FM_MP && (o.nb == 1 || o.nb == 4);
+  return o.method == METHOD_HARMONIC && o.hN <= FM_MAXN && (o.nb == 1 || o.nb == 4);
 }
 
 void allocate_pass_buffers(Plan &plan) {
@@ -827,17 +939,24 @@ void m2l_dense_level(Plan &plan, int l) {
     const int32_t t0 = li.chunk_t[k], nt = li.chunk_t[k + 1] - t0;
     if (npk == 0 || nt == 0) continue;
     if (fused) {
-      const float *reps32r = plan.hl[l]->reps32r.p;
+      const bf16x8 *ops = reinterpret_cast<const bf16x8 *>(plan.hl[l]->repsb.p);
+      const uint32_t *g8 = reinterpret_cast<const uint32_t *>(o.gsel8.p), *f8 = reinterpret_cast<const uint32_t *>(o.fsel8.p);
       const int ppt = FM_COLS / nb;
       for (int c = 0; c < o.nclass; c++) ca.to[c + 1] = ca.to[c] + (ca.co[c + 1] - ca.co[c] + ppt - 1) / ppt;
       const int32_t ntiles = ca.to[o.nclass];
-      const unsigned grid = (unsigned)std::min<int64_t>(ntiles, 4 * 256);
-      if (nb == 4)
-        k_class_m2l32<4><<<grid, FM_TB, 0, s>>>(plan.Yc32.p, plan.Mp.p, Ns, N, reps32r, li.csrc.p, li.cfar.p, o.gsel.p,
-                                                o.fsel.p, o.offs.p, ca, ntiles, li.ctgt.p);
-      else
-        k_class_m2l32<1><<<grid, FM_TB, 0, s>>>(plan.Yc32.p, plan.Mp.p, Ns, N, reps32r, li.csrc.p, li.cfar.p, o.gsel.p,
-                                                o.fsel.p, o.offs.p, ca, ntiles, li.ctgt.p);
+      const unsigned grid = (unsigned)std::min<int64_t>(ntiles, 2 * 256);   // two workgroups per CU
+      auto go = [&](auto NB, auto KB) {
+        k_class_m2l32<decltype(NB)::value, decltype(KB)::value><<<grid, FM_TB, 0, s>>>(
+            plan.Yc32.p, plan.Mp.p, Ns, N, ops, li.csrc.p, li.cfar.p, g8, f8, o.offs.p, ca, ntiles, li.ctgt.p);
+      };
+      auto kb = [&](auto NB) {
+        if (N <= 32) go(NB, std::integral_constant<int, 1>{});
+        else if (N <= 64) go(NB, std::integral_constant<int, 2>{});
+        else if (N <= 96) go(NB, std::integral_constant<int, 3>{});
+        else go(NB, std::integral_constant<int, 4>{});
+      };
+      if (nb == 4) kb(std::integral_constant<int, 4>{});
+      else kb(std::integral_constant<int, 1>{});
       FFMM_LAUNCH_CHECK();
       if (nbN % 4 == 0) {
         const unsigned bt4 = (unsigned)std::min(1024, (nbN / 4 + 63) / 64 * 64);

@@ -273,9 +273,7 @@ __global__ void __launch_bounds__(64 * SpBoxes<T>::NB) k_spec_inverse(const type
 // matrix cores (26%) in turn, the fetches running at 1.5 TB/s.
 // ---------------------------------------------------------------------------
 constexpr int HM_TILE = 16;          // sibling groups per tile: the matrix instructions' columns
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // The levels 2 .. L-1 of a plan: first node, first sibling group and first tile of each.
 struct SpLevels {
@@ -523,15 +521,6 @@ __device__ __forceinline__ double swap_rows(double x) {
   const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0xB1, 0xF, 0xF, false);
   const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0xB1, 0xF, 0xF, false);
   return __hiloint2double(hi, lo);
-}
-
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pack_bf16(f32x2 v) {   // round to nearest even, both at once
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
-}
-__device__ __forceinline__ f32x2 unpack_bf16(uint32_t b) {
-  return f32x2{__uint_as_float(b << 16), __uint_as_float(b & 0xffff0000u)};
 }
 
 struct HadArgs {
