@@ -442,6 +442,8 @@ int64_t compact_flags_u8(Context &ctx, const uint8_t *flag, int32_t *idx, int64_
 // the device has stored its value
 void arm_slots(Context &ctx, int first, int n);
 int64_t read_slot(Context &ctx, int slot);
+// where the host knows the count already
+void compact_flags_u8_known(Context &ctx, const uint8_t *flag, int32_t *idx, int64_t n);
 // the count into the context's pinned slot `slot` (0 .. 62) by the stream, no synchronisation
 void compact_flags_u8_async(Context &ctx, const uint8_t *flag, int32_t *idx, int64_t n, int slot);
 void set_pinned(Context &ctx, int slot, int64_t v);

@@ -135,6 +135,17 @@ int64_t compact_flags_u8(Context &ctx, const uint8_t *flag, int32_t *idx, int64_
   return poll_slot(ctx, POLL_SLOT);
 }
 
+// the same where the host knows the count: nothing is read back
+void compact_flags_u8_known(Context &ctx, const uint8_t *flag, int32_t *idx, int64_t n) {
+  if (n <= 0) return;
+  rocprim::counting_iterator<int32_t> it(0);
+  size_t bytes = 0;
+  FFMM_HIP(rocprim::select(nullptr, bytes, it, flag, idx, (int32_t *)nullptr, (size_t)n, ctx.stream));
+  size_t off = (bytes + 255) & ~size_t(255);
+  char *t = static_cast<char *>(scratch(ctx, off + 256));
+  FFMM_HIP(rocprim::select(t, bytes, it, flag, idx, reinterpret_cast<int32_t *>(t + off), (size_t)n, ctx.stream));
+}
+
 __global__ void k_copy_count_slot(const int32_t *__restrict__ dcount, int64_t *__restrict__ host) {
   if (threadIdx.x == 0) host[0] = dcount[0];
 }
