@@ -24,7 +24,7 @@ constexpr double C4PI = 0.07957747154594767;   // 1 / (4 pi), as 1 / (4 * Float6
 // (src/device_passes.jl:378-403).  pM[k, q] = sum_j tau_j K(x_j - c, y_k).
 // ---------------------------------------------------------------------------
 constexpr int S2M_TB = 256;
-constexpr int S2M_KP = 6;   // check points per thread: ceil(1352 / 256)
+constexpr int S2M_KP = 6;   // check points per thread; blockIdx.y: blocks of S2M_TB S2M_KP points (1,736 points at p = 9)
 
 __global__ void __launch_bounds__(S2M_TB) k_s2m(const int32_t *__restrict__ nodes, const double *__restrict__ centers,
                                                 int64_t nn, const int32_t *__restrict__ level,
@@ -38,11 +38,11 @@ __global__ void __launch_bounds__(S2M_TB) k_s2m(const int32_t *__restrict__ node
   const int node = nodes[q];
   const double c0 = centers[node], c1 = centers[nn + node], c2 = centers[2 * nn + node];
   const double s = lam[level[node]];
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, k0 = blockIdx.y * (S2M_TB * S2M_KP);
   double acc[S2M_KP], y0[S2M_KP], y1[S2M_KP], y2[S2M_KP];
 #pragma unroll
   for (int m = 0; m < S2M_KP; m++) {
-    int k = t + S2M_TB * m;
+    int k = k0 + t + S2M_TB * m;
     acc[m] = 0.0;
     if (k < Nl) {
       y0[m] = surf[k] * s;
@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(S2M_TB) k_s2m(const int32_t *__restrict__ node
   }
 #pragma unroll
   for (int m = 0; m < S2M_KP; m++) {
-    int k = t + S2M_TB * m;
+    int k = k0 + t + S2M_TB * m;
     if (k < Nl) pM[q * Nl + k] = acc[m];
   }
 }
@@ -97,12 +97,12 @@ __global__ void __launch_bounds__(S2M_TB) k_s2m32(const int32_t *__restrict__ no
   const int node = nodes[q];
   const double c0 = centers[node], c1 = centers[nn + node], c2 = centers[2 * nn + node];
   const double s = lam[level[node]];
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, k0 = blockIdx.y * (S2M_TB * S2M_KP);
   double acc[S2M_KP];
   float y0[S2M_KP], y1[S2M_KP], y2[S2M_KP];
 #pragma unroll
   for (int m = 0; m < S2M_KP; m++) {
-    const int k = t + S2M_TB * m;
+    const int k = k0 + t + S2M_TB * m;
     acc[m] = 0.0;
     if (k < Nl) {
       y0[m] = (float)(surf[k] * s);
@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(S2M_TB) k_s2m32(const int32_t *__restrict__ no
   }
 #pragma unroll
   for (int m = 0; m < S2M_KP; m++) {
-    const int k = t + S2M_TB * m;
+    const int k = k0 + t + S2M_TB * m;
     if (k < Nl) pM[q * Nl + k] = C4PI * acc[m];
   }
 }
@@ -866,12 +866,13 @@ void upward_pass(Plan &plan) {
     // S2M into check potentials, then UC2E, M = pinv_scale V diag(invS) (Uh pM)
     // (src/device_passes.jl:496-502), as two GEMMs over all of them.  pinv_scale = lam[l]
     // is a power of two, applied exactly in the scatter.
+    const dim3 g((unsigned)nq, (unsigned)((Nl + S2M_TB * S2M_KP - 1) / (S2M_TB * S2M_KP)));
     if (plan.precision == FFMM_PREC_MIXED)
-      k_s2m32<<<(unsigned)nq, S2M_TB, 0, s>>>(nodes, plan.centers.p, plan.nnodes, plan.level.p, plan.lam_d.p,
+      k_s2m32<<<g, S2M_TB, 0, s>>>(nodes, plan.centers.p, plan.nnodes, plan.level.p, plan.lam_d.p,
                                               o.large.p, Nl, plan.plo.p, plan.phi.p, plan.sx.p, plan.sy.p, plan.sz.p,
                                               plan.tau.p, plan.pM.p);
     else
-      k_s2m<<<(unsigned)nq, S2M_TB, 0, s>>>(nodes, plan.centers.p, plan.nnodes, plan.level.p, plan.lam_d.p, o.large.p,
+      k_s2m<<<g, S2M_TB, 0, s>>>(nodes, plan.centers.p, plan.nnodes, plan.level.p, plan.lam_d.p, o.large.p,
                                             Nl, plan.plo.p, plan.phi.p, plan.sx.p, plan.sy.p, plan.sz.p, plan.tau.p,
                                             plan.pM.p);
     FFMM_LAUNCH_CHECK();

@@ -84,3 +84,15 @@ def test_harmonic_blocks_vs_oracle(kernel, p):
     u_ref = oracle_for(m, cache, pts, 10, tree.perm)[0].matvec(d)
     u_ref = u_ref.reshape(u.shape)
     assert np.max(np.abs(u - u_ref)) < 1e-11 * np.max(np.abs(u_ref))
+
+
+def test_odd_order_of_many_check_points():
+    """p = 9: 1,736 check points, more than one block of the general S2M; conditioned as p = 10."""
+    import ffmm
+    rng = np.random.default_rng(9)
+    pts, tau = rng.random((1500, 3)), rng.standard_normal(1500)
+    m = ffmm.CubeKernelIndependent(ffmm.Laplace3D(), p=9)
+    cache = ffmm.OperatorCache(m)
+    u = ffmm.DevicePlan(m, pts, ppl=25, bbox=BOX, cache=cache).matvec(tau).cpu().numpy()
+    u_ref = O.FMM(cache.host_operators(), pts, 25, BOX[0], BOX[1]).matvec(tau)
+    assert np.max(np.abs(u - u_ref)) < 1e-10 * np.max(np.abs(u_ref))
