@@ -51,17 +51,18 @@ def interaction_counts(tree, nleaf_targets=None):
 
 
 def gemm_shapes(plan, ops, mixed: bool):
-    """The GEMMs of one step of the cube method, in launch order: (name, m, n, k, type,
-    flop, library: run by the BLAS library).  Per step: UC2E as two FP64 factors over the childless sourced nodes of
+    """The dense products of one step of the cube method, in launch order: (name, m, n, k, type,
+    flop, library).  They size the step's work in its plain form; where the reflections of the
+    surfaces serve (even orders up to 10) the library runs them as eight blocks of an eighth of
+    the size, M2M in FP64.  Per step: UC2E as two FP64 factors over the childless sourced nodes of
     levels 2 and below, M2M per level (FP32 in the mixed form, in calls of at most 10,240
     columns) from level L-2 up to 2, L2L
     per level (FP64) from level 3 down, DC2E as two FP64 factors over the leaves."""
     Ns, Nl, L = ops.nsmall, ops.nlarge, plan.nlevels
     nq_up, nq_dn = int(plan.level_s2m[2:].sum()), int(plan.level_leaves[2:].sum())
     ru, rd = ops.P_up.rank, ops.P_down.rank
-    # ranks 241..304: UC2E's first factor runs inside k_s2m_uc2e (S2M fused with it), not as
-    # a library GEMM; with 240 < Ns <= 304 (r_dn likewise), UC2E's second factor and DC2E's
-    # first run as k_gemm_cols
+    # the labels of the p = 8 products name the kernels of an earlier form; they stay, so that
+    # records compare
     fused = 241 <= ru <= 304
     cols_up, cols_dn = 240 < Ns <= 304, 240 < rd <= 304
     out = [("UC2E Uh" + (" (in k_s2m_uc2e)" if fused else ""), ru, nq_up, Nl, "f64"),
@@ -615,16 +616,15 @@ def main():
     pairs = int(plan.level_pairs.sum())
     if args.m2l == "spectral":
         # the dominant kernel: the Hadamard products of the spectral M2L, one launch per
-        # level (mixed: the union kernel, then on some levels the per-group kernel for the
-        # tiles the union staging does not take, timed together); algorithmic work = far
-        # pairs x 2304 frequencies x 8 flops (a complex multiply-add), over the summed
-        # HIP-event time on the plan's stream
-        nfreq = 9 * 16 * 16
+        # level; algorithmic work = far pairs x 1,688 frequencies (a real length-15 transform
+        # without the conjugates) x 8 flops (a complex multiply-add), over the summed HIP-event
+        # time on the plan's stream
+        nfreq = (15 ** 3 + 1) // 2
         flops = float(pairs) * nfreq * 8
         t_k = stages["hadamard"] * 1e-3
         peak = PEAK_FP64_TFLOPS if args.precision == "f64" else PEAK_FP32_MFMA_TFLOPS
-        kname = ("k_spec_hadamard_union + k_spec_hadamard_mfma" if args.precision == "mixed"
-                 else "k_spec_hadamard<double, 8>") + " (spectral M2L Hadamard products)"
+        kname = ("k_spec_hadamard<false>" if args.precision == "mixed"
+                 else "k_spec_hadamard<true>") + " (spectral M2L Hadamard products)"
     else:
         flops = float(pairs) * 2 * m.nsurface ** 2
         t_k = stages["m2l"] * 1e-3
@@ -635,12 +635,12 @@ def main():
     roofline = {"bound": "mfma", "achieved": achieved, "peak": peak, "unit": "TFLOP/s", "frac": achieved / peak,
                 "traffic": traffic_from_profile(kname, args), "kernel": kname, "launches": nlaunch,
                 "avg_launch_ms": 1e3 * t_k / max(nlaunch, 1), "flops_per_launch": flops / max(nlaunch, 1),
-                "note": ("FP32 MFMA kernels (v_mfma_f32_16x16x4_f32) against the dense FP32 MFMA peak, a "
-                         "launch being one level (the union kernel, then the per-group kernel for the "
-                         "tiles it does not take); achieved counts the far pairs' products only, the "
-                         "MFMAs also multiply the near pairs' zero table rows of each 8 x 8 block and the "
-                         "missing colleagues' zero boxes") if args.precision == "mixed" else
-                        "VALU FMA kernel: MI355X's vector FP64 and FP64-MFMA peaks are both 78.6 TFLOP/s",
+                "note": ("FP32 operands as three bfloat16 pieces, six products each on "
+                         "v_mfma_f32_16x16x32_bf16, against the dense FP32 MFMA peak; achieved counts the far "
+                         "pairs' products only, the instructions also multiply the near pairs' zero table rows "
+                         "of each 8 x 8 block and the missing colleagues' zero boxes")
+                if args.precision == "mixed" else
+                        "v_mfma_f64_16x16x4: MI355X's vector FP64 and FP64-MFMA peaks are both 78.6 TFLOP/s",
                 "eval_sources": {"flops": flops_eval, "ms": stages["eval_sources"],
                                  "achieved_tflops": flops_eval / (stages["eval_sources"] * 1e-3) / 1e12}}
 
