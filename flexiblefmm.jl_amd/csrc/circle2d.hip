@@ -400,28 +400,45 @@ __global__ void k_c2_fill(double *__restrict__ a, int64_t n) {
 }
 
 // M2L (m2l_level!, src/fmm.jl:100-127, by target): pL[:, t] += sum over the target's
-// pairs of M2L[f] Mp[:, s]; one wave per target, lane k the entry k of the product
-__global__ void __launch_bounds__(C2_TB) k_c2_m2l(double *__restrict__ pL, const double *__restrict__ Mp,
-                                               const int32_t *__restrict__ ptr, const int32_t *__restrict__ src,
-                                               const int32_t *__restrict__ far, const double *__restrict__ A,
-                                               int n) {
-  __shared__ double m[C2_TB];
-  const int64_t t = blockIdx.x;
-  const int32_t p0 = ptr[t], p1 = ptr[t + 1];
-  if (p0 == p1) return;
-  const int k = threadIdx.x;
-  double acc = 0.0;
-  for (int32_t e = p0; e < p1; e++) {
-    const int64_t s = src[e];
+// pairs of M2L[f] Mp[:, s]; one wave per target, lane k the entry k of the product.
+// A pair reads its offset's matrix (28.8 KB at n = 60), 3.9 GB through the L2 at 10^5 points:
+// that and the chain of n dependent products bounded one wave per workgroup.  Here a
+// workgroup's four waves take the same child slot of four consecutive sibling groups, whose
+// lists run through the same offsets, in step, so that a matrix is read into the L1 once for
+// the four where the lists agree; four chains per sum, the next expansion in flight.
+constexpr int C2_MW = 4;
+__global__ void __launch_bounds__(C2_MW *C2_TB) k_c2_m2l(double *__restrict__ pL, const double *__restrict__ Mp,
+                                                         const int32_t *__restrict__ ptr, const int32_t *__restrict__ src,
+                                                         const int32_t *__restrict__ far, const double *__restrict__ A,
+                                                         int n, int64_t nl) {
+  __shared__ double m[2][C2_MW][C2_TB];
+  __shared__ int32_t cnt[C2_MW];
+  const int w = threadIdx.x / C2_TB, k = threadIdx.x % C2_TB;
+  const int64_t t = (int64_t)(blockIdx.x / 4) * (4 * C2_MW) + 4 * w + blockIdx.x % 4;
+  const int32_t p0 = t < nl ? ptr[t] : 0, np = t < nl ? ptr[t + 1] - p0 : 0;
+  if (k == 0) cnt[w] = np;
+  __syncthreads();
+  const int32_t rounds = max(max(cnt[0], cnt[1]), max(cnt[2], cnt[3]));
+  double c[4] = {0.0, 0.0, 0.0, 0.0};
+  double x = np > 0 && k < n ? Mp[(int64_t)src[p0] * n + k] : 0.0;
+  for (int32_t r = 0; r < rounds; r++) {
+    double(&mr)[C2_TB] = m[r & 1][w];
+    mr[k] = x;
     __syncthreads();
-    if (k < n) m[k] = Mp[s * n + k];
-    __syncthreads();
-    if (k < n) {
-      const double *__restrict__ a = A + (int64_t)far[e] * n * n + k;
-      for (int i = 0; i < n; i++) acc = fma(a[(int64_t)i * n], m[i], acc);
+    if (r < np) {
+      if (r + 1 < np && k < n) x = Mp[(int64_t)src[p0 + r + 1] * n + k];
+      if (k < n) {
+        const double *__restrict__ a = A + (int64_t)far[p0 + r] * n * n + k;
+        int i = 0;
+#pragma unroll 4
+        for (; i + 4 <= n; i += 4)
+#pragma unroll
+          for (int j = 0; j < 4; j++) c[j] = fma(a[(int64_t)(i + j) * n], mr[i + j], c[j]);
+        for (; i < n; i++) c[0] = fma(a[(int64_t)i * n], mr[i], c[0]);
+      }
     }
   }
-  if (k < n) pL[t * n + k] += acc;
+  if (np > 0 && k < n) pL[t * n + k] += (c[0] + c[1]) + (c[2] + c[3]);
 }
 
 // evaluate_target (src/evaluate.jl:37-58), Potential: the L2T of the target's leaf
@@ -564,7 +581,8 @@ static void build_expansions(Plan2 &p, const double *tau) {
       gemm(ctx, C2_NCH * n, (int)ng, n, p.ops[l - 1].L2L.p, C2_NCH * n, p.work.p, n, pL, C2_NCH * n);
     }
     if (!p.h.src[l].empty()) {
-      k_c2_m2l<<<(unsigned)nl, C2_TB, 0, s>>>(pL, p.Mp.p, p.ptr[l].p, p.src[l].p, p.far[l].p, o.M2L.p, n);
+      k_c2_m2l<<<(unsigned)(4 * ((nl + 4 * C2_MW - 1) / (4 * C2_MW))), C2_MW * C2_TB, 0, s>>>(
+          pL, p.Mp.p, p.ptr[l].p, p.src[l].p, p.far[l].p, o.M2L.p, n, nl);
       FFMM_LAUNCH_CHECK();
     }
     const int64_t nq = (int64_t)p.leaves_h[l].size();
