@@ -402,43 +402,38 @@ __global__ void k_c2_fill(double *__restrict__ a, int64_t n) {
 // M2L (m2l_level!, src/fmm.jl:100-127, by target): pL[:, t] += sum over the target's
 // pairs of M2L[f] Mp[:, s]; one wave per target, lane k the entry k of the product.
 // A pair reads its offset's matrix (28.8 KB at n = 60), 3.9 GB through the L2 at 10^5 points:
-// that and the chain of n dependent products bounded one wave per workgroup.  Here a
-// workgroup's four waves take the same child slot of four consecutive sibling groups, whose
-// lists run through the same offsets, in step, so that a matrix is read into the L1 once for
-// the four where the lists agree; four chains per sum, the next expansion in flight.
-constexpr int C2_MW = 4;
-__global__ void __launch_bounds__(C2_MW *C2_TB) k_c2_m2l(double *__restrict__ pL, const double *__restrict__ Mp,
-                                                         const int32_t *__restrict__ ptr, const int32_t *__restrict__ src,
-                                                         const int32_t *__restrict__ far, const double *__restrict__ A,
-                                                         int n, int64_t nl) {
-  __shared__ double m[2][C2_MW][C2_TB];
-  __shared__ int32_t cnt[C2_MW];
-  const int w = threadIdx.x / C2_TB, k = threadIdx.x % C2_TB;
-  const int64_t t = (int64_t)(blockIdx.x / 4) * (4 * C2_MW) + 4 * w + blockIdx.x % 4;
-  const int32_t p0 = t < nl ? ptr[t] : 0, np = t < nl ? ptr[t + 1] - p0 : 0;
-  if (k == 0) cnt[w] = np;
-  __syncthreads();
-  const int32_t rounds = max(max(cnt[0], cnt[1]), max(cnt[2], cnt[3]));
+// that and the chain of dependent products bound it, so each sum runs in four chains with
+// the next expansion in flight.  A wave is a workgroup of its own and waits for no other:
+// four targets in step behind a barrier per pair share a matrix only where their lists run
+// through the same offsets, which those of adaptive trees do not.  Potential at the sources and
+// at half as many targets, one chain / four in step / this (us): uniform 160k points, 60 per
+// circle 1,777 / 1,672 / 1,569; mixture 160k, 40 per circle 2,059 / 2,148 / 1,940.
+__global__ void __launch_bounds__(C2_TB) k_c2_m2l(double *__restrict__ pL, const double *__restrict__ Mp,
+                                               const int32_t *__restrict__ ptr, const int32_t *__restrict__ src,
+                                               const int32_t *__restrict__ far, const double *__restrict__ A, int n) {
+  __shared__ double m[2][C2_TB];   // alternating: one barrier per pair
+  const int64_t t = blockIdx.x;
+  const int32_t p0 = ptr[t], p1 = ptr[t + 1];
+  if (p0 == p1) return;
+  const int k = threadIdx.x;
   double c[4] = {0.0, 0.0, 0.0, 0.0};
-  double x = np > 0 && k < n ? Mp[(int64_t)src[p0] * n + k] : 0.0;
-  for (int32_t r = 0; r < rounds; r++) {
-    double(&mr)[C2_TB] = m[r & 1][w];
-    mr[k] = x;
-    __syncthreads();
-    if (r < np) {
-      if (r + 1 < np && k < n) x = Mp[(int64_t)src[p0 + r + 1] * n + k];
-      if (k < n) {
-        const double *__restrict__ a = A + (int64_t)far[p0 + r] * n * n + k;
-        int i = 0;
+  double x = k < n ? Mp[(int64_t)src[p0] * n + k] : 0.0;
+  for (int32_t e = p0; e < p1; e++) {
+    double(&me)[C2_TB] = m[(e - p0) & 1];
+    me[k] = x;
+    lds_barrier();                 // of one wave: the next expansion's load stays in flight
+    if (k < n) {
+      if (e + 1 < p1) x = Mp[(int64_t)src[e + 1] * n + k];
+      const double *__restrict__ a = A + (int64_t)far[e] * n * n + k;
+      int i = 0;
 #pragma unroll 4
-        for (; i + 4 <= n; i += 4)
+      for (; i + 4 <= n; i += 4)
 #pragma unroll
-          for (int j = 0; j < 4; j++) c[j] = fma(a[(int64_t)(i + j) * n], mr[i + j], c[j]);
-        for (; i < n; i++) c[0] = fma(a[(int64_t)i * n], mr[i], c[0]);
-      }
+        for (int j = 0; j < 4; j++) c[j] = fma(a[(int64_t)(i + j) * n], me[i + j], c[j]);
+      for (; i < n; i++) c[0] = fma(a[(int64_t)i * n], me[i], c[0]);
     }
   }
-  if (np > 0 && k < n) pL[t * n + k] += (c[0] + c[1]) + (c[2] + c[3]);
+  if (k < n) pL[t * n + k] += (c[0] + c[1]) + (c[2] + c[3]);
 }
 
 // evaluate_target (src/evaluate.jl:37-58), Potential: the L2T of the target's leaf
@@ -581,8 +576,7 @@ static void build_expansions(Plan2 &p, const double *tau) {
       gemm(ctx, C2_NCH * n, (int)ng, n, p.ops[l - 1].L2L.p, C2_NCH * n, p.work.p, n, pL, C2_NCH * n);
     }
     if (!p.h.src[l].empty()) {
-      k_c2_m2l<<<(unsigned)(4 * ((nl + 4 * C2_MW - 1) / (4 * C2_MW))), C2_MW * C2_TB, 0, s>>>(
-          pL, p.Mp.p, p.ptr[l].p, p.src[l].p, p.far[l].p, o.M2L.p, n, nl);
+      k_c2_m2l<<<(unsigned)nl, C2_TB, 0, s>>>(pL, p.Mp.p, p.ptr[l].p, p.src[l].p, p.far[l].p, o.M2L.p, n);
       FFMM_LAUNCH_CHECK();
     }
     const int64_t nq = (int64_t)p.leaves_h[l].size();

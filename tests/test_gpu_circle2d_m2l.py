@@ -1,7 +1,6 @@
-"""The circle method's M2L with four targets per workgroup: circles of 4 to 64 points (with and
-without a remainder of the four chains, a full wave), levels whose sibling groups are not a
-multiple of four, ragged lists, against the oracle's FMM on the same tree (1e-11: FP64 sums in
-another order, through the pseudo-inverses)."""
+"""The circle method's M2L: circles of 4 to 64 points (with and without a remainder of the four
+chains, a full wave), empty and ragged lists, against the oracle's FMM on the same tree
+(1e-11: FP64 sums in another order, through the pseudo-inverses)."""
 import numpy as np
 import pytest
 
