@@ -406,21 +406,27 @@ int ffmm_opcache_put_cube(ffmm_opcache cache, double w_ref, const double *small,
     o.r_up = r_up;
     o.r_dn = r_dn;
     o.nclass = nclass;
-    // even orders with full-rank pseudo-inverses: every point array in orbit order from here on
+    // even orders with full-rank pseudo-inverses, where the operators are those that the blocks
+    // stand for: every point array in orbit order from here on
     o.sym = false;
     o.embed_h = cube_embed(o.p);
     std::vector<double> small_o, large_o, M2M_o, L2L_o, cls_o;
     std::vector<int32_t> idx_o;
     std::vector<int8_t> sgn_o;
-    const bool sym = sym_fits(o.p, o.pc, Ns, r_up, r_dn) && on_lattice(small, o.p) && on_lattice(large, o.pc);
+    SymFactors fac;
+    bool sym = sym_fits(o.p, o.pc, Ns, r_up, r_dn) && on_lattice(small, o.p) && on_lattice(large, o.pc) &&
+               sym_matches(o, small, large, {Uh_up, invS_up, V_up, Uh_dn, invS_dn, V_dn, M2M, L2L});
     if (sym) {
       o.sym_small = sym_orbits(o.p);
       o.sym_large = sym_orbits(o.pc);
-      const std::vector<int32_t> &ps = o.sym_small, &pl = o.sym_large;
+      for (const int32_t i : o.sym_small) small_o.insert(small_o.end(), small + 3 * i, small + 3 * i + 3);
+      for (const int32_t i : o.sym_large) large_o.insert(large_o.end(), large + 3 * i, large + 3 * i + 3);
+      sym = sym_factor(o, small_o, large_o, fac);
+    }
+    if (sym) {
+      const std::vector<int32_t> &ps = o.sym_small;
       std::vector<int32_t> ip(Ns);
       for (int i = 0; i < Ns; i++) ip[ps[i]] = i;
-      for (int i = 0; i < Ns; i++) small_o.insert(small_o.end(), small + 3 * ps[i], small + 3 * ps[i] + 3);
-      for (int i = 0; i < Nl; i++) large_o.insert(large_o.end(), large + 3 * pl[i], large + 3 * pl[i] + 3);
       M2M_o.resize((size_t)Ns * NCHILD * Ns);
       L2L_o.resize(M2M_o.size());
       cls_o.resize((size_t)nclass * Ns * Ns);
@@ -461,7 +467,7 @@ int ffmm_opcache_put_cube(ffmm_opcache cache, double w_ref, const double *small,
     std::vector<float> soa32(soa.begin(), soa.end());
     o.large32.upload(soa32.data(), soa32.size(), s);
     if (sym) {
-      sym_setup(o, small_o, large_o, M2M_o, L2L_o);
+      sym_setup(o, fac, large_o, M2M_o, L2L_o);
     } else {
       o.Uh_up.upload(Uh_up, (size_t)r_up * Nl, s);
       o.Uh_dn.upload(Uh_dn, (size_t)r_dn * Ns, s);

@@ -491,8 +491,16 @@ void m2l_spectral_level(Plan &plan, int l);
 // ---- the cube method's translations by symmetric blocks (sym.hip) ----
 std::vector<int32_t> sym_orbits(int n);
 bool sym_fits(int p, int pc, int Ns, int r_up, int r_dn);
-void sym_setup(OpCache &o, const std::vector<double> &small, const std::vector<double> &large,
-               const std::vector<double> &M2M, const std::vector<double> &L2L);
+struct SymGiven {                 // the operators as given (full ranks; column major)
+  const double *Uh_up, *invS_up, *V_up, *Uh_dn, *invS_dn, *V_dn, *M2M, *L2L;
+};
+bool sym_matches(const OpCache &o, const double *small, const double *large, const SymGiven &g);
+struct SymFactors {               // per block K_chi = U diag(S) V^T
+  std::vector<double> U[8], S[8], V[8];
+};
+bool sym_factor(const OpCache &o, const std::vector<double> &small, const std::vector<double> &large, SymFactors &f);
+void sym_setup(OpCache &o, const SymFactors &f, const std::vector<double> &large, const std::vector<double> &M2M,
+               const std::vector<double> &L2L);
 // fewer childless sourced nodes than this: S2M as a kernel of its own (a workgroup per node
 // and 64 orbits), else inside UC2E (16 nodes per workgroup)
 constexpr int64_t SYM_SPLIT_NODES = 8192;

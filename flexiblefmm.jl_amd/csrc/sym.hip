@@ -728,11 +728,14 @@ std::vector<int32_t> sym_orbits(int n) {
 }
 
 // One-sided Jacobi: A (m x n, column major, m >= n) = U diag(s) V^T; A becomes U, V n x n.
-static void jacobi_svd(std::vector<double> &A, int m, int n, std::vector<double> &s, std::vector<double> &V) {
+// False when U's columns are not orthogonal to 1e-12 after 60 sweeps, or A has no full rank.
+static bool jacobi_svd(std::vector<double> &A, int m, int n, std::vector<double> &s, std::vector<double> &V) {
   V.assign((size_t)n * n, 0.0);
   for (int i = 0; i < n; i++) V[(size_t)i * n + i] = 1.0;
+  double worst = 0.0;            // the largest cosine that the last sweep met
   for (int sweep = 0; sweep < 60; sweep++) {
     bool done = true;
+    worst = 0.0;
     for (int i = 0; i < n - 1; i++)
       for (int j = i + 1; j < n; j++) {
         double *x = &A[(size_t)i * m], *y = &A[(size_t)j * m];
@@ -744,6 +747,7 @@ static void jacobi_svd(std::vector<double> &A, int m, int n, std::vector<double>
         }
         if (std::abs(ab) <= 1e-15 * std::sqrt(aa * bb)) continue;
         done = false;
+        worst = std::max(worst, std::abs(ab) / std::sqrt(aa * bb));
         const double z = (bb - aa) / (2.0 * ab);
         const double tn = (z >= 0.0 ? 1.0 : -1.0) / (std::abs(z) + std::sqrt(1.0 + z * z));
         const double cs = 1.0 / std::sqrt(1.0 + tn * tn), sn = cs * tn;
@@ -764,8 +768,10 @@ static void jacobi_svd(std::vector<double> &A, int m, int n, std::vector<double>
     double q = 0.0;
     for (int k = 0; k < m; k++) q += A[(size_t)i * m + k] * A[(size_t)i * m + k];
     s[i] = std::sqrt(q);
-    for (int k = 0; k < m; k++) A[(size_t)i * m + k] = s[i] > 0.0 ? A[(size_t)i * m + k] / s[i] : 0.0;
+    if (!(s[i] > 0.0)) return false;
+    for (int k = 0; k < m; k++) A[(size_t)i * m + k] /= s[i];
   }
+  return worst <= 1e-12;
 }
 
 static inline double chi_sign(int chi, int h) { return __builtin_popcount(chi & h) & 1 ? -1.0 : 1.0; }
@@ -776,11 +782,134 @@ bool sym_fits(int p, int pc, int Ns, int r_up, int r_dn) {
   return (p == 2 || p == 4 || p == 6 || p == 8 || p == 10) && pc % 2 == 0 && r_up == Ns && r_dn == Ns;
 }
 
-// The blocks, from the surfaces and the folded M2M / L2L in orbit order (M2M: Ns x 8 Ns,
-// L2L: 8 Ns x Ns, column major), averaged over the reflections (their own rounding is not
-// symmetric).
-void sym_setup(OpCache &o, const std::vector<double> &small, const std::vector<double> &large,
-               const std::vector<double> &M2M, const std::vector<double> &L2L) {
+// Whether the given operators are those the blocks stand for, to rounding; a cache given
+// others (a regularised inverse, say) keeps them, dense.  Checked on vectors, against the
+// Laplace matrix K from the small to the large surface, with everything in the given order:
+//   the factors of P_up and P_down are singular value decompositions of K and K^T: U S V^T x
+//     = K x to 1e-13 s_1 |x|, U and V orthonormal to 1e-12;
+//   M2M and L2L commute with the reflections, M2M in the potentials K M2M x, L2L on
+//     potentials K^T y, to 1e-11 (their own entries keep the inverses' amplified rounding,
+//     1e-7 at p = 8, which neither sees).
+// Operators of level_operators measure 5e-16, 4e-15 and at most 1.6e-13 (p = 2 .. 10, d = 0.01
+// .. 0.6).
+bool sym_matches(const OpCache &o, const double *small, const double *large, const SymGiven &g) {
+  const int Ns = o.Ns, Nl = o.Nl, C = NCHILD;
+  const std::vector<int32_t> os = sym_orbits(o.p);
+  uint64_t seed = 1;
+  auto vec = [&](int n) {
+    std::vector<double> x(n);
+    for (double &v : x) {
+      seed = seed * 6364136223846793005ull + 1442695040888963407ull;
+      v = (double)(int64_t)(seed >> 11) / 4503599627370496.0 - 1.0;
+    }
+    return x;
+  };
+  // y = A x and A^T x, A (m x n, column major)
+  auto mul = [](const double *A, int m, int n, const std::vector<double> &x) {
+    std::vector<double> y(m, 0.0);
+    for (int j = 0; j < n; j++)
+      for (int i = 0; i < m; i++) y[i] += A[(size_t)j * m + i] * x[j];
+    return y;
+  };
+  auto tmul = [](const double *A, int m, int n, const std::vector<double> &x) {
+    std::vector<double> y(n, 0.0);
+    for (int j = 0; j < n; j++)
+      for (int i = 0; i < m; i++) y[j] += A[(size_t)j * m + i] * x[i];
+    return y;
+  };
+  auto norm = [](const std::vector<double> &x) {
+    double q = 0.0;
+    for (double v : x) q += v * v;
+    return std::sqrt(q);
+  };
+  auto differ = [](const std::vector<double> &x, const std::vector<double> &y) {
+    double q = 0.0;
+    for (size_t i = 0; i < x.size(); i++) q += (x[i] - y[i]) * (x[i] - y[i]);
+    return std::sqrt(q);
+  };
+  std::vector<double> K((size_t)Nl * Ns);
+  for (int r = 0; r < Ns; r++)
+    for (int k = 0; k < Nl; k++) {
+      double r2 = 0.0;
+      for (int d = 0; d < 3; d++) {
+        const double e = large[3 * (size_t)k + d] - small[3 * (size_t)r + d];
+        r2 += e * e;
+      }
+      K[(size_t)r * Nl + k] = C4PI / std::sqrt(r2);
+    }
+  double s1 = 0.0;
+  for (int i = 0; i < Ns; i++)
+    if (!(g.invS_up[i] > 0.0 && g.invS_dn[i] > 0.0)) return false;
+    else s1 = std::max(s1, 1.0 / g.invS_up[i]);
+  for (int n = 0; n < 4; n++) {
+    const std::vector<double> x = vec(Ns), y = vec(Nl), Kx = mul(K.data(), Nl, Ns, x), Ky = tmul(K.data(), Nl, Ns, y);
+    // P_up = V S^-1 U^T: U^T is Uh_up (Ns x Nl), V is V_up (Ns x Ns)
+    std::vector<double> t = tmul(g.V_up, Ns, Ns, x);
+    if (!(differ(mul(g.V_up, Ns, Ns, t), x) <= 1e-12 * norm(x))) return false;
+    for (int i = 0; i < Ns; i++) t[i] /= g.invS_up[i];
+    const std::vector<double> u = tmul(g.Uh_up, Ns, Nl, t);
+    if (!(differ(mul(g.Uh_up, Ns, Nl, u), t) <= 1e-12 * norm(t))) return false;
+    if (!(differ(u, Kx) <= 1e-13 * s1 * norm(x))) return false;
+    // P_down = V S^-1 U^T of K^T = U S V^T: V_dn (Nl x Ns), Uh_dn (Ns x Ns)
+    t = tmul(g.V_dn, Nl, Ns, y);
+    for (int i = 0; i < Ns; i++) t[i] /= g.invS_dn[i];
+    const std::vector<double> w = tmul(g.Uh_dn, Ns, Ns, t);
+    if (!(differ(mul(g.Uh_dn, Ns, Ns, w), t) <= 1e-12 * norm(t))) return false;
+    if (!(differ(tmul(g.V_dn, Nl, Ns, mul(g.V_dn, Nl, Ns, x)), x) <= 1e-12 * norm(x))) return false;
+    if (!(differ(w, Ky) <= 1e-13 * s1 * norm(y))) return false;
+  }
+  for (int f = 1; f < 8; f <<= 1) {   // the reflection of one coordinate
+    std::vector<int32_t> at(Ns);
+    for (int i = 0; i < Ns; i++) at[os[i]] = os[i ^ f];
+    auto points = [&](const std::vector<double> &a) {
+      std::vector<double> b(a.size());
+      for (int i = 0; i < Ns; i++) b[at[i]] = a[i];
+      return b;
+    };
+    auto children = [&](const std::vector<double> &a) {
+      std::vector<double> b(a.size());
+      for (int c = 0; c < C; c++)
+        for (int i = 0; i < Ns; i++) b[(size_t)(c ^ f) * Ns + at[i]] = a[(size_t)c * Ns + i];
+      return b;
+    };
+    const std::vector<double> x = vec(C * Ns);
+    std::vector<double> a = mul(K.data(), Nl, Ns, points(mul(g.M2M, Ns, C * Ns, x)));
+    if (!(differ(a, mul(K.data(), Nl, Ns, mul(g.M2M, Ns, C * Ns, children(x)))) <= 1e-11 * norm(a))) return false;
+    const std::vector<double> l = tmul(K.data(), Nl, Ns, vec(Nl));
+    a = children(mul(g.L2L, C * Ns, Ns, l));
+    if (!(differ(a, mul(g.L2L, C * Ns, Ns, points(l))) <= 1e-11 * norm(a))) return false;
+  }
+  return true;
+}
+
+// The blocks' singular value decompositions from the surfaces in orbit order; false when one
+// of them did not converge.
+bool sym_factor(const OpCache &o, const std::vector<double> &small, const std::vector<double> &large, SymFactors &f) {
+  const int nr = o.Ns / 8, nk = o.Nl / 8;
+  for (int chi = 0; chi < 8; chi++) {
+    // K_chi[k, r] = sum_h chi(h) K(x_(k, h), y_(r, 0))
+    std::vector<double> &U = f.U[chi];
+    U.assign((size_t)nk * nr, 0.0);
+    for (int r = 0; r < nr; r++)
+      for (int k = 0; k < nk; k++)
+        for (int h = 0; h < 8; h++) {
+          double r2 = 0.0;
+          for (int d = 0; d < 3; d++) {
+            const double e = large[3 * (size_t)(8 * k) + d] * ((h >> d) & 1 ? -1.0 : 1.0) - small[3 * (size_t)(8 * r) + d];
+            r2 += e * e;
+          }
+          U[(size_t)r * nk + k] += chi_sign(chi, h) * C4PI / std::sqrt(r2);
+        }
+    if (!jacobi_svd(U, nk, nr, f.S[chi], f.V[chi])) return false;
+  }
+  return true;
+}
+
+// The operators' blocks, from those factors and the folded M2M / L2L in orbit order (M2M: Ns
+// x 8 Ns, L2L: 8 Ns x Ns, column major), averaged over the reflections (their own rounding
+// is not symmetric).
+void sym_setup(OpCache &o, const SymFactors &f, const std::vector<double> &large, const std::vector<double> &M2M,
+               const std::vector<double> &L2L) {
   const int nr = o.Ns / 8, nk = o.Nl / 8, Ns = o.Ns;
   const int R = (nr + 15) / 16 * 16, KP = (nk + SY_K - 1) / SY_K * SY_K, KP2 = (Ns + SY_K - 1) / SY_K * SY_K;
   const int K4 = (nr + 3) / 4 * 4;
@@ -794,20 +923,7 @@ void sym_setup(OpCache &o, const std::vector<double> &small, const std::vector<d
   std::vector<double> u1(8 * (size_t)KP * R + 16 * R, 0.0), u2(8 * (size_t)(R + 16) * R + 16 * R, 0.0), d1 = u2,
       d2(8 * (size_t)K4 * KP, 0.0), mm(8 * (size_t)KP2 * R + 16 * R, 0.0), ll(8 * (size_t)K4 * KP2, 0.0);
   for (int chi = 0; chi < 8; chi++) {
-    // K_chi[k, r] = sum_h chi(h) K(x_(k, h), y_(r, 0))
-    std::vector<double> U((size_t)nk * nr, 0.0), S, V;
-    for (int r = 0; r < nr; r++)
-      for (int k = 0; k < nk; k++)
-        for (int h = 0; h < 8; h++) {
-          double r2 = 0.0;
-          for (int d = 0; d < 3; d++) {
-            const double x = (h >> d) & 1 ? -rep[(size_t)d * nk + k] : rep[(size_t)d * nk + k];
-            const double e = x - small[3 * (size_t)(8 * r) + d];
-            r2 += e * e;
-          }
-          U[(size_t)r * nk + k] += chi_sign(chi, h) * C4PI / std::sqrt(r2);
-        }
-    jacobi_svd(U, nk, nr, S, V);
+    const std::vector<double> &U = f.U[chi], &S = f.S[chi], &V = f.V[chi];
     for (int i = 0; i < nr; i++) {
       for (int k = 0; k < nk; k++) {
         u1[((size_t)chi * KP + k) * R + i] = U[(size_t)i * nk + k];

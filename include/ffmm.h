@@ -116,7 +116,12 @@ int ffmm_opcache_destroy(ffmm_opcache cache);
  *   far offsets, and per offset the signed permutation idx (Ns x 316, 0-based), sgn (Ns x 316)
  *   with M2L_f m = P_f A_rep (P_f^T m), (P^T m)[i] = sgn[i] m[idx[i]];
  *   tables: the spectral kernel tables, 316 x (2p)(2p)(p+1) complex (interleaved re, im),
- *   or NULL to disable the spectral M2L. */
+ *   or NULL to disable the spectral M2L.
+ * Where P_up and P_down are full-rank pseudo-inverses of the Laplace matrix between the
+ * surfaces, and these and M2M, L2L keep the reflections of the cube (p = 2, 4, 6, 8 or 10,
+ * pc even), they are applied as 8 blocks each, factored here; both hold to rounding
+ * (1e-13 of the largest singular value; 1e-11 of the potentials that M2M and L2L give) or
+ * the operators are applied as given. */
 int ffmm_opcache_put_cube(ffmm_opcache cache, double w_ref, const double *small, const double *large,
                           int r_up, const double *Uh_up, const double *invS_up, const double *V_up,
                           int r_dn, const double *Uh_dn, const double *invS_dn, const double *V_dn,

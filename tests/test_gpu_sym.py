@@ -96,3 +96,44 @@ def test_odd_order_of_many_check_points():
     u = ffmm.DevicePlan(m, pts, ppl=25, bbox=BOX, cache=cache).matvec(tau).cpu().numpy()
     u_ref = O.FMM(cache.host_operators(), pts, 25, BOX[0], BOX[1]).matvec(tau)
     assert np.max(np.abs(u - u_ref)) < 1e-10 * np.max(np.abs(u_ref))
+
+
+@pytest.mark.parametrize("precision", ["f64", "mixed"])
+@pytest.mark.parametrize("p,given", [(4, "scaled inverse"), (8, "regularised inverse"), (8, "scaled inverse down"),
+                                     (4, "M2M of one child"), (8, "L2L of one child"), (8, "truncated"), (8, "odd pc")])
+def test_given_operators_are_applied(p, given, precision):
+    """Even orders whose operators are not those of the blocks (a scaled or regularised inverse
+    of full rank, a truncated one, translations without the reflections' symmetry, check
+    surfaces of an odd order) are applied as given: against the oracle with the same operators,
+    to the tolerances of test_blocks_vs_oracle."""
+    import ffmm
+    print(f"[sym] given operators: {given} p={p} {precision}", flush=True)
+    rng = np.random.default_rng(p)
+    n = 2000
+    pts = rng.random((n, 3))
+    pts[: n // 3] = 0.4 + 0.05 * rng.random((n // 3, 3))
+    tau = rng.standard_normal(n)
+    kw = {"truncated": dict(pinv_rtol=1e-8), "odd pc": dict(pc=15)}.get(given, {})
+    m = ffmm.CubeKernelIndependent(ffmm.Laplace3D(), p=p, **kw)
+    cache = ffmm.OperatorCache(m)
+    cache.fit_box(pts.min(0), pts.max(0), BOX)
+    o = cache.host_operators()
+    if given == "scaled inverse":
+        o.P_up.invS *= 2.0
+    elif given == "scaled inverse down":
+        o.P_down.invS *= 0.5
+    elif given == "regularised inverse":
+        s = 1.0 / o.P_up.invS
+        o.P_up.invS[:] = s / (s * s + (1e-6 * s[0]) ** 2)
+    elif given == "M2M of one child":
+        o.M2M[:, : o.nsmall] *= 1.25
+    elif given == "L2L of one child":
+        o.L2L[: o.nsmall] *= 1.25
+    elif given == "truncated":
+        assert o.P_up.rank < o.nsmall
+    u = ffmm.DevicePlan(m, pts, ppl=20, bbox=BOX, cache=cache, precision=precision).matvec(tau).cpu().numpy()
+    u_ref = O.FMM(o, pts, 20, BOX[0], BOX[1]).matvec(tau)
+    if precision == "mixed":
+        assert np.linalg.norm(u - u_ref) < 2e-6 * np.linalg.norm(u_ref)
+    else:
+        assert np.max(np.abs(u - u_ref)) < 1e-11 * np.max(np.abs(u_ref))
