@@ -850,6 +850,7 @@ static void plan_finish(Plan &p) {
     p.khat.upload(kh.data(), p.L, ctx.stream);
   }
   node_leafslots(p);
+  near_work(p);
   {
     StageTimer tm(p, 1);
     build_lists(p);
@@ -857,6 +858,7 @@ static void plan_finish(Plan &p) {
   allocate_pass_buffers(p);
   if (p.m2l == FFMM_M2L_SPECTRAL) spectral_prepare(p);
   ctx.sync();
+  near_work_read(p);
 }
 
 void plan_init(Plan &p, Context &ctx, OpCache &o, const double *xyz, int64_t n, int ppl, const double origin[3],
@@ -1595,6 +1597,15 @@ int ffmm_plan_spectral_tiles(ffmm_plan plan, int64_t *staged, int64_t *per_group
       staged[l] = per_group[l] = 0;
       if (l < p.L) spectral_tile_counts(p, l, staged[l], per_group[l]);
     }
+  });
+}
+
+int ffmm_plan_near_work(ffmm_plan plan, double out[3]) {
+  return guard([&] {
+    if (!plan || !out) fail(FFMM_ERR_ARGUMENT, "null argument");
+    out[0] = plan->c.near_sum;
+    out[1] = plan->c.near_max;
+    out[2] = (double)plan->c.near_leaves;
   });
 }
 

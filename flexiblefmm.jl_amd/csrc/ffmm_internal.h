@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <functional>
 #include <map>
@@ -378,6 +380,10 @@ struct Plan {
   // node lists per level (concatenated): childless sourced nodes, real leaves
   std::vector<int64_t> s2m_off, leaf_off;   // L + 1 offsets
   DBuf<int32_t> s2m_nodes, leaf_nodes;
+  // plans of fewer than EVAL_WIDE_LEAVES leaves: those with points, and the sum and the
+  // largest of points x near sources over them
+  int64_t near_leaves = 0;
+  double near_sum = 0.0, near_max = 0.0;
   std::vector<LevelLists> lists;
   // expansions
   DBuf<double> Mp, Pl, Lc;   // Ns x n, Ns x n, Nl x nleaves
@@ -604,17 +610,37 @@ __device__ __forceinline__ f32x2 unpack_bf16(uint32_t b) {
   return f32x2{__uint_as_float(b << 16), __uint_as_float(b & 0xffff0000u)};
 }
 
-// The evaluation kernels take one workgroup per leaf, of one wave or, where there are few
-// leaves, of four: with one wave each, few leaves leave the card's 1,024 SIMDs idle or with
-// too few waves to hide a tile's loads, and the largest leaves end last.  Measured, one wave
-// / four (ms):
-//   cube mixed, 20 points a leaf    9,997 leaves .109 / .079   29,037 leaves .128 / .165
-//   cube mixed, 200 points a leaf   3,676 leaves 2.19 / .84    12,937 leaves 2.90 / 1.43
-//   cube FP64, 64 points a leaf       960 leaves .241 / .091   22,149 leaves .603 / .566
-//   Stokes mixed, 64 points a leaf  1,030 leaves .486 / .172   10,130 .705 / .479   22,226 .785 / .902
-//   Yukawa mixed, 64 points a leaf    981 leaves .305 / .114    5,286 .333 / .295   10,130 .379 / .562
-// Yukawa turns first: the exponential leaves less to hide, the lanes' weights fill the LDS.
+// The evaluation kernels take one workgroup per leaf, of one wave or of four.  One wave each
+// leaves the card's 1,024 SIMDs idle where there are few leaves, and lets the largest leaves end
+// last; four waves cost their barriers and the sum of their parts, which small leaves do not
+// pay back.  So the largest leaf's share of the work decides: four waves where it is more than
+// 1 / share, a leaf's work being its targets x near sources (near_work: those of the sources,
+// in proportion for other targets) and 3,200 such pairs for what does not depend on them.
+// Measured at the sources, one wave / four (ms; leaves, points a leaf; p = 8, Yukawa 10):
+//                  uniform, 4,096    uniform, 4,096    density ~ x^-1/3 an axis
+//                  leaves of 6       of 32             6,014 of 2.4    5,937 of 15    10,424 of 15
+//   cube FP64        .084 / .071       .404 / .315     .061 / .061     .334 / .202    .404 / .326
+//   Laplace mixed    .035 / .039       .236 / .184     .035 / .040     .359 / .137    .357 / .161
+//   Stokes mixed     .061 / .100       .381 / .320     .059 / .110     .476 / .212    .464 / .349
+//   Stokes FP64      .096 / .146       .627 / .477     .086 / .170     .501 / .326    .556 / .565
+//   Yukawa mixed     .055 / .111       .319 / .367     .050 / .136     .309 / .270    .303 / .464
+// Over 140 plans and 0.5 to 16 targets a leaf the rule loses 0.5 to 1.5% on average to the
+// better of the two, 1.3 times at most; the number of leaves alone lost up to 2.7 times.
 constexpr int64_t EVAL_WIDE_LEAVES = 16384, EVAL_WIDE_LEAVES_YUKAWA = 6144;
+inline bool eval_wide(const Plan &plan, int64_t ntargets) {
+  constexpr double FIXED = 3200.0;
+  const OpCache &o = *plan.ops;
+  const bool yukawa = o.kernel == FFMM_KERNEL_YUKAWA;
+  const double share = o.method == METHOD_CUBE                ? 3600.0
+                       : yukawa                               ? 450.0
+                       : o.kernel == FFMM_KERNEL_LAPLACE      ? 3200.0
+                       : plan.precision == FFMM_PREC_MIXED    ? 1400.0
+                                                              : 900.0;
+  const double f = (double)ntargets / (double)plan.N;
+  const double leaves = (double)std::min(plan.near_leaves, ntargets);
+  return plan.leaf_off[plan.L] < (yukawa ? EVAL_WIDE_LEAVES_YUKAWA : EVAL_WIDE_LEAVES) &&
+         leaves * FIXED + plan.near_sum * f < share * (plan.near_max * f + FIXED);
+}
 
 // sums of the replicas of each of ntp targets (thread t: target t % ntp) into the threads
 // below ntp; red: 4 EVT doubles (not used for one wave).  Synchronises a block of four waves.
@@ -711,7 +737,10 @@ size_t plan_bytes(const Plan &p);
 
 // ---- harmonic methods (harmonic.hip) ----
 void harmonic_s2m_level(Plan &plan, int l);
-void launch_eval_harmonic(Plan &plan, const EvalArgs &a, int output);
+void launch_eval_harmonic(Plan &plan, const EvalArgs &a, int output, bool wide);
+// the near field's work by leaf, queued; near_work_read after the stream's next synchronisation
+void near_work(Plan &plan);
+void near_work_read(Plan &plan);
 
 // ---- timing ----
 struct StageTimer {

@@ -787,26 +787,25 @@ static void launch_eval_harm(const OpCache &o, const EvalArgs &a, int output, un
   FFMM_LAUNCH_CHECK();
 }
 template <class T>
-static void launch_eval_harm(const OpCache &o, const EvalArgs &a, int output, int64_t nleaves, hipStream_t s) {
+static void launch_eval_harm(const OpCache &o, const EvalArgs &a, int output, bool wide, int64_t nleaves, hipStream_t s) {
   // per workgroup: the leaf's expansion and, Yukawa, each lane's radial weights
   auto lds = [&](int evt) {
     return ((size_t)o.Ns * sizeof(T) + 7) / 8 * 8 +
            (o.kernel == FFMM_KERNEL_YUKAWA ? 2 * sizeof(double) * evt * (o.p + 2) : 0);
   };
-  // four waves where there are few leaves, unless the weights of 256 lanes (p > 12) fill the LDS
-  const int64_t wide = o.kernel == FFMM_KERNEL_YUKAWA ? EVAL_WIDE_LEAVES_YUKAWA : EVAL_WIDE_LEAVES;
-  if (nleaves < wide && lds(256) <= 64 * 1024)
+  // not four waves where the weights of 256 lanes take more than 64 KiB (Yukawa, p > 13)
+  if (wide && lds(256) <= 64 * 1024)
     launch_eval_harm<T, 256>(o, a, output, (unsigned)nleaves, lds(256), s);
   else
     launch_eval_harm<T, 64>(o, a, output, (unsigned)nleaves, lds(64), s);
 }
 
 // the mixed form evaluates in FP32 (k_eval_harm<float>), the FP64 form in FP64
-void launch_eval_harmonic(Plan &plan, const EvalArgs &a, int output) {
+void launch_eval_harmonic(Plan &plan, const EvalArgs &a, int output, bool wide) {
   const int64_t nleaves = plan.leaf_off[plan.L];
   if (nleaves == 0) return;
-  if (plan.precision == FFMM_PREC_MIXED) launch_eval_harm<float>(*plan.ops, a, output, nleaves, plan.ctx->stream);
-  else launch_eval_harm<double>(*plan.ops, a, output, nleaves, plan.ctx->stream);
+  if (plan.precision == FFMM_PREC_MIXED) launch_eval_harm<float>(*plan.ops, a, output, wide, nleaves, plan.ctx->stream);
+  else launch_eval_harm<double>(*plan.ops, a, output, wide, nleaves, plan.ctx->stream);
 }
 
 }  // namespace ffmm

@@ -799,6 +799,13 @@ class DevicePlan:
              b.ctypes.data_as(ctypes.c_void_p), self.nlevels)
         return a, b
 
+    def near_work(self):
+        """The sum and the largest of points × near sources over the leaves with points, and
+        the number of these (zeros for a plan of 16,384 leaves or more)."""
+        out = np.zeros(3)
+        call("ffmm_plan_near_work", self._h, out.ctypes.data_as(ctypes.c_void_p))
+        return out
+
     def stage_times(self) -> dict:
         ms = (ctypes.c_double * 9)()
         call("ffmm_plan_stage_times", self._h, ms, 9)
