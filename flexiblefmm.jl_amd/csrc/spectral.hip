@@ -893,10 +893,10 @@ void spectral_prepare(Plan &plan) {
   read_slot(ctx, L);   // the compaction's own count: its slot is free again
 }
 
-// The tiles of level l staged whole, and those cut into parts (the mixed form).
+// The tiles of level l staged whole, and those cut into parts (a plan with spectral tiles).
 bool spectral_tile_counts(const Plan &plan, int l, int64_t &staged, int64_t &cut) {
   staged = cut = 0;
-  if (plan.precision != FFMM_PREC_MIXED || l + 1 >= (int)plan.spec_tile0.size() || plan.spec_nsub[l] == 0) return false;
+  if (plan.m2l != FFMM_M2L_SPECTRAL || l + 1 >= (int)plan.spec_tile0.size() || plan.spec_nsub[l] == 0) return false;
   std::vector<uint8_t> fl((size_t)HU_SUB * (plan.spec_tile0[l + 1] - plan.spec_tile0[l]));
   FFMM_HIP(hipMemcpy(fl.data(), plan.spec_flag.p + HU_SUB * plan.spec_tile0[l], fl.size(), hipMemcpyDeviceToHost));
   for (size_t i = 0; i < fl.size(); i += HU_SUB) {

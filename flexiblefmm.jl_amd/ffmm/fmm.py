@@ -792,8 +792,8 @@ class DevicePlan:
         return M.T, Pl.T, Lc.T
 
     def spectral_tiles(self):
-        """Per level, the tiles of the mixed spectral M2L's Hadamard products run by the
-        kernel staging each tile's distinct colleague boxes, and by the per-group kernel."""
+        """Per level, the tiles of 16 sibling groups of the spectral M2L's Hadamard products
+        whose distinct colleague boxes are staged whole, and those cut into subtiles."""
         a, b = np.zeros(self.nlevels, dtype=np.int64), np.zeros(self.nlevels, dtype=np.int64)
         call("ffmm_plan_spectral_tiles", self._h, a.ctypes.data_as(ctypes.c_void_p),
              b.ctypes.data_as(ctypes.c_void_p), self.nlevels)

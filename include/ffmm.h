@@ -314,8 +314,8 @@ int ffmm_plan_set_tol(ffmm_plan plan, double tol);
 int ffmm_plan_stage_times(ffmm_plan plan, double *ms, int n);
 /* Per level l < n, the tiles (16 sibling groups each) of the spectral M2L's Hadamard
  * products whose distinct colleague boxes are staged whole (staged[l]) and those cut into
- * subtiles (per_group[l]); zeros for other plans.  No reference counterpart: a diagnostic. */
-int ffmm_plan_spectral_tiles(ffmm_plan plan, int64_t *staged, int64_t *per_group, int n);
+ * subtiles (cut[l]); zeros for other plans.  No reference counterpart: a diagnostic. */
+int ffmm_plan_spectral_tiles(ffmm_plan plan, int64_t *staged, int64_t *cut, int n);
 /* The near field's work of the leaves with points, which the evaluation's launch is chosen by:
  * out[0] the sum and out[1] the largest of a leaf's points x near sources, out[2] the number
  * of such leaves; zeros for a plan of 16,384 leaves or more.  No reference counterpart: a
