@@ -59,12 +59,13 @@ def test_sources_beyond_the_lds_stage(precision):
 
 
 @pytest.mark.parametrize("kernel,p", [("laplace", 2), ("laplace", 5), ("laplace", 10), ("yukawa", 7), ("laplace", 13),
-                                      ("stokes", 3), ("stokes", 10), ("laplace", 16)])
+                                      ("stokes", 3), ("stokes", 10), ("laplace", 16), ("laplace", 18), ("laplace", 19),
+                                      ("stokes", 18), ("laplace", 20), ("stokes", 20)])
 def test_harmonic_blocks_vs_oracle(kernel, p):
     """M2M and L2L by reflection parity against the harmonic oracle's dense operators on the
-    same tree (1e-11, as tests/test_gpu_harmonic.py): one to three row tiles, expansions of
-    one to five chunks of 64 entries, one and four blocks, groups of 16 and of 4 columns with
-    missing ones."""
+    same tree (1e-11, as tests/test_gpu_harmonic.py): one to four row tiles, expansions of
+    one to seven chunks of 64 entries, one and four blocks, groups of 16 and of 4 columns with
+    missing ones; p = 20, whose largest block has more than 64 entries, keeps the dense form."""
     import ffmm
     from test_gpu_harmonic import oracle_for
     print(f"[sym] harmonic {kernel} p={p}", flush=True)

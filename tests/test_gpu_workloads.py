@@ -107,9 +107,9 @@ def test_mixture_mixed_spectral_targets(mixture):
 
 def test_mixture_400k_mixed_spectral_both_hadamard_kernels():
     """400,000 Gaussian-mixture sources, mixed precision, spectral M2L. At this size a few
-    tiles of 16 sibling groups name more than 200 distinct colleague boxes, so the
-    Hadamard products run in both kernels (the one staging each tile's boxes once, and
-    the per-group one for those tiles); the potential at the sources within 2e-6
+    tiles of 16 sibling groups name more than 192 distinct colleague boxes, so the
+    Hadamard products run on tiles staged whole and on tiles cut into subtiles; the
+    potential at the sources within 2e-6
     (max-norm) of the oracle's FP64 FMM on the same tree, and within the 1e-6 rel L2
     gate of the FP64 direct sum on 3,000 sampled sources."""
     import ffmm
@@ -119,11 +119,11 @@ def test_mixture_400k_mixed_spectral_both_hadamard_kernels():
     tau = W.charges(n, seed=1)
     m = ffmm.CubeKernelIndependent(ffmm.Laplace3D(), p=8)
     cache = ffmm.OperatorCache(m)
-    print(f"[workloads] mixture n={n}, mixed spectral, both Hadamard kernels", flush=True)
+    print(f"[workloads] mixture n={n}, mixed spectral, whole and cut tiles", flush=True)
     plan = ffmm.DevicePlan(m, pts, ppl=64, bbox=BOX, cache=cache, precision="mixed", m2l="spectral")
-    staged, per_group = plan.spectral_tiles()
-    print(f"[workloads] tiles staged {staged.tolist()}, per group {per_group.tolist()}", flush=True)
-    assert staged.sum() > 0 and per_group.sum() > 0
+    staged, cut = plan.spectral_tiles()
+    print(f"[workloads] tiles staged whole {staged.tolist()}, cut {cut.tolist()}", flush=True)
+    assert staged.sum() > 0 and cut.sum() > 0
     plan.build_expansions(tau)
     u = plan.evaluate_at_sources(ffmm.Potential).cpu().numpy()
     tree = plan.download_tree()
@@ -135,19 +135,21 @@ def test_mixture_400k_mixed_spectral_both_hadamard_kernels():
 
 
 def test_mixture_3m_mixed_m2m_in_column_chunks():
-    """3,000,000 Gaussian-mixture sources: some levels have more than 10,240 sibling
-    groups, so the mixed form's FP32 M2M runs in several column chunks there.  The
-    potential at every source agrees with the plain FP64 plan on the same points (which
-    makes one M2M call per level) to the mixed form's 1e-6 rel L2."""
+    """3,000,000 Gaussian-mixture sources and truncated pseudo-inverses (rank 292 of 296), whose
+    operators stay dense: some levels have more than 10,240 sibling groups, so the mixed
+    form's FP32 M2M runs in several column chunks there.  The potential at every source
+    agrees with the plain FP64 plan on the same points (which makes one M2M call per level)
+    to the mixed form's 1e-6 rel L2."""
     import ffmm
     from ffmm import workloads as W
     n = 3_000_000
     pts = W.gaussian_mixture(n, seed=5)
     tau = W.charges(n, seed=6)
-    m = ffmm.CubeKernelIndependent(ffmm.Laplace3D(), p=8)
+    m = ffmm.CubeKernelIndependent(ffmm.Laplace3D(), p=8, pinv_rtol=1e-9)
     cache = ffmm.OperatorCache(m)
     print(f"[workloads] mixture n={n}, mixed vs FP64, chunked M2M", flush=True)
     mixed = ffmm.DevicePlan(m, pts, ppl=64, bbox=BOX, cache=cache, precision="mixed", m2l="spectral")
+    assert cache.host_operators().P_up.rank < m.nsurface
     groups = np.asarray(mixed.level_count) // 8
     print(f"[workloads] sibling groups per level {groups.tolist()}", flush=True)
     assert groups[3:].max() > 10240
