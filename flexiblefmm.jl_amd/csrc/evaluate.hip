@@ -359,6 +359,7 @@ void near_work_read(Plan &plan) {
 static void launch_eval(Plan &plan, EvalArgs &a, int output, int64_t ntargets) {
   const int64_t nleaves = plan.leaf_off[plan.L];
   if (nleaves == 0) return;
+  check_operators(plan);
   const bool wide = eval_wide(plan, ntargets);
   if (plan.ops->method == METHOD_HARMONIC) {
     launch_eval_harmonic(plan, a, output, wide);

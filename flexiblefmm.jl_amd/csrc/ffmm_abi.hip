@@ -1160,6 +1160,7 @@ void plan_capture(Plan &p, int nd, int output, const double *dens) {
 
 void plan_replay(Plan &p, const double *dens, double *out) {
   if (!p.gexec) fail(FFMM_ERR_STATE, "the plan holds no captured pass sequence");
+  check_operators(p);
   set_device(*p.ctx);
   hipStream_t s = p.ctx->stream;
   FFMM_HIP(hipMemcpyAsync(p.gin.p, dens, sizeof(double) * p.g_nd * p.N, hipMemcpyDefault, s));

@@ -384,6 +384,9 @@ struct Plan {
   // largest of points x near sources over them
   int64_t near_leaves = 0;
   double near_sum = 0.0, near_max = 0.0;
+  // the form and the largest rank of the cube operators that the buffers were made for
+  bool sym = false;
+  int rank = 0;
   std::vector<LevelLists> lists;
   // expansions
   DBuf<double> Mp, Pl, Lc;   // Ns x n, Ns x n, Nl x nleaves
@@ -484,6 +487,7 @@ void allocate_pass_buffers(Plan &plan);
 // a[0 .. n) = v on the context's stream (a kernel: no memset node in a captured graph)
 void fill_f64(Context &ctx, double *a, int64_t n, double v);
 void gather_inputs(Plan &plan, const double *tau, int sorted);
+void check_operators(const Plan &plan);
 void upward_pass(Plan &plan);
 void downward_pass(Plan &plan);
 void m2l_dense_level(Plan &plan, int l);

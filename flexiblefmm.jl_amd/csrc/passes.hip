@@ -773,6 +773,8 @@ void allocate_pass_buffers(Plan &plan) {
       plan.Mup.resize((size_t)Ns * nq);
     }
   }
+  plan.sym = o.sym;
+  plan.rank = std::max(o.r_up, o.r_dn);
   if (!o.sym) {
     plan.tM.resize((size_t)Ns * ng);
     if (o.method == METHOD_CUBE && plan.precision == FFMM_PREC_MIXED) {
@@ -813,7 +815,16 @@ void gather_inputs(Plan &plan, const double *tau, int sorted) {
 }
 
 // upward pass: src/device_passes.jl:523-547
+// whether the plan's buffers and expansions are of the form of its cache's operators, which may
+// have been put again since
+void check_operators(const Plan &plan) {
+  const OpCache &o = *plan.ops;
+  if (o.method == METHOD_CUBE && (plan.sym != o.sym || std::max(o.r_up, o.r_dn) > plan.rank))
+    fail(FFMM_ERR_STATE, "the cache's operators were replaced by others of another form since the plan was made");
+}
+
 void upward_pass(Plan &plan) {
+  check_operators(plan);
   Context &ctx = *plan.ctx;
   OpCache &o = *plan.ops;
   hipStream_t s = ctx.stream;

@@ -121,7 +121,9 @@ int ffmm_opcache_destroy(ffmm_opcache cache);
  * surfaces, and these and M2M, L2L keep the reflections of the cube (p = 2, 4, 6, 8 or 10,
  * pc even), they are applied as 8 blocks each, factored here; both hold to rounding
  * (1e-13 of the largest singular value; 1e-11 of the potentials that M2M and L2L give) or
- * the operators are applied as given. */
+ * the operators are applied as given.  Operators put again while plans of the cache exist
+ * serve these plans if they are applied in the same form with no larger rank; else the
+ * plans' passes fail with FFMM_ERR_STATE. */
 int ffmm_opcache_put_cube(ffmm_opcache cache, double w_ref, const double *small, const double *large,
                           int r_up, const double *Uh_up, const double *invS_up, const double *V_up,
                           int r_dn, const double *Uh_dn, const double *invS_dn, const double *V_dn,

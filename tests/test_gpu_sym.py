@@ -138,3 +138,40 @@ def test_given_operators_are_applied(p, given, precision):
         assert np.linalg.norm(u - u_ref) < 2e-6 * np.linalg.norm(u_ref)
     else:
         assert np.max(np.abs(u - u_ref)) < 1e-11 * np.max(np.abs(u_ref))
+
+
+def test_operators_put_again(monkeypatch):
+    """Operators put again into a cache that a plan was made with: of the same form, the plan
+    serves them; of the other form (here a scaled inverse, applied as given), the plan's
+    passes, its evaluation and its captured replay are refused, and a new plan is right."""
+    import ffmm
+    from ffmm import fmm as F
+    rng = np.random.default_rng(4)
+    pts, tau = rng.random((1500, 3)), rng.standard_normal(1500)
+    m = ffmm.CubeKernelIndependent(ffmm.Laplace3D(), p=4)
+    cache = ffmm.OperatorCache(m)
+    plan = ffmm.DevicePlan(m, pts, ppl=20, bbox=BOX, cache=cache).capture()
+    u = plan.matvec(tau).cpu().numpy()
+    h, call = cache.device(0), F.call
+
+    def put_again(name, *args):
+        if name == "ffmm_opcache_create":
+            args[-1]._obj.value = h.value
+        else:
+            call(name, *args)
+
+    def again():
+        cache._device.clear()
+        monkeypatch.setattr(F, "call", put_again)
+        cache.device(0)
+        monkeypatch.setattr(F, "call", call)
+    again()
+    assert np.array_equal(plan.matvec(tau).cpu().numpy(), u)
+    cache.host_operators().P_up.invS *= 2.0
+    again()
+    for step in (plan.evaluate_at_sources, lambda: plan.replay(tau), lambda: plan.build_expansions(tau)):
+        with pytest.raises(ffmm.DeviceError, match="replaced"):
+            step()
+    v = ffmm.DevicePlan(m, pts, ppl=20, bbox=BOX, cache=cache).matvec(tau).cpu().numpy()
+    v_ref = O.FMM(cache.host_operators(), pts, 20, BOX[0], BOX[1]).matvec(tau)
+    assert np.max(np.abs(v - v_ref)) < 1e-11 * np.max(np.abs(v_ref))
