@@ -523,8 +523,7 @@ int ffmm_opcache_put_cube(ffmm_opcache cache, double w_ref, const double *small,
         int x = u % 7 - 3, y = (u / 7) % 7 - 3, z = u / 49 - 3;
         far_index[u] = std::max(std::abs(x), std::max(std::abs(y), std::abs(z))) >= 2 ? nf++ : -1;
       }
-      // one more row, all near: the FP64 Hadamard's table copy reads past the last candidate
-      std::vector<int16_t> pf((NCOLL * NCHILD + 1) * NCHILD, (int16_t)-1);
+      std::vector<int16_t> pf(NCOLL * NCHILD * NCHILD, (int16_t)-1);
       for (int k = 0; k < NCOLL; k++)
         for (int c = 0; c < NCHILD; c++)
           for (int a = 0; a < NCHILD; a++) {

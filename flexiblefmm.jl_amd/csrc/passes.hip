@@ -728,7 +728,9 @@ static void gemm(Context &ctx, int m, int n, int k, double alpha, const double *
                           &beta, C, ldc));
 }
 
-constexpr int64_t M2M32_CHUNK = 10240;   // columns per call of the mixed form's M2M GEMM
+// columns per call of the mixed form's dense M2M (p = 8 with a truncated inverse or an odd
+// number of check points per edge; measured there, the odd orders take the same)
+constexpr int64_t M2M32_CHUNK = 10240;
 
 static void gemm32(Context &ctx, int m, int n, int k, const float *A, int lda, const float *B, int ldb, float *C,
                    int ldc) {
@@ -775,13 +777,18 @@ void allocate_pass_buffers(Plan &plan) {
   }
   plan.sym = o.sym;
   plan.rank = std::max(o.r_up, o.r_dn);
-  if (!o.sym) {
+  // M2M and L2L as dense products (harmonic levels that do not split; Yukawa's are not known yet)
+  const bool harm = o.method == METHOD_HARMONIC;
+  bool dense = !harm && !o.sym;
+  if (harm)
+    for (const HarmonicLevel *h : plan.hl) dense |= !h || !h->sym_m2m.p;
+  if (dense) {
     plan.tM.resize((size_t)Ns * ng);
-    if (o.method == METHOD_CUBE && plan.precision == FFMM_PREC_MIXED) {
+    if (!harm && plan.precision == FFMM_PREC_MIXED) {
       plan.Mp32.resize((size_t)Ns * plan.nnodes);
       plan.tM32.resize((size_t)Ns * ng);
     }
-    plan.G.resize((size_t)Ns * std::max(nq, ng));
+    plan.G.resize((size_t)Ns * (harm ? ng : std::max(nq, ng)));
   }
   int64_t pmax = 1;
   for (auto &li : plan.lists) pmax = std::max(pmax, li.chunk_max);
