@@ -739,6 +739,7 @@ int ffmm_opcache_put_class_factors(ffmm_opcache cache, double tol, const int32_t
     if (!(tol > 0 && tol < 1)) fail(FFMM_ERR_ARGUMENT, "tol must lie in (0, 1)");
     auto f = std::make_unique<ClassFactors>();
     f->tol = tol;
+    f->sym = o.sym;
     int64_t tot = 0;
     for (int c = 0; c < o.nclass; c++) {
       if (ranks[c] < 1 || ranks[c] > o.Ns) fail(FFMM_ERR_ARGUMENT, "a class rank lies outside 1:Ns");

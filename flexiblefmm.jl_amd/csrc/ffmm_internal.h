@@ -330,6 +330,7 @@ struct ClassFactors {
   std::vector<int> rank;        // k_c per class
   std::vector<int64_t> off;     // first entry of A_c (and of Bt_c) in A, Bt
   int kmax = 0;
+  bool sym = false;             // rows of A and columns of Bt in orbit order
   DBuf<double> A, Bt;
   DBuf<float> A32, Bt32;
 };

@@ -822,11 +822,12 @@ void gather_inputs(Plan &plan, const double *tau, int sorted) {
 }
 
 // upward pass: src/device_passes.jl:523-547
-// whether the plan's buffers and expansions are of the form of its cache's operators, which may
-// have been put again since
+// whether the plan's buffers and expansions, and its low-rank factors, are of the form of its
+// cache's operators, which may have been put again since
 void check_operators(const Plan &plan) {
   const OpCache &o = *plan.ops;
-  if (o.method == METHOD_CUBE && (plan.sym != o.sym || std::max(o.r_up, o.r_dn) > plan.rank))
+  if (o.method != METHOD_CUBE) return;
+  if (plan.sym != o.sym || std::max(o.r_up, o.r_dn) > plan.rank || (plan.lowrank && plan.lowrank->sym != o.sym))
     fail(FFMM_ERR_STATE, "the cache's operators were replaced by others of another form since the plan was made");
 }
 

@@ -152,6 +152,7 @@ def test_operators_put_again(monkeypatch):
     cache = ffmm.OperatorCache(m)
     plan = ffmm.DevicePlan(m, pts, ppl=20, bbox=BOX, cache=cache).capture()
     u = plan.matvec(tau).cpu().numpy()
+    cache.class_factors(0, 1e-6)
     h, call = cache.device(0), F.call
 
     def put_again(name, *args):
@@ -172,6 +173,10 @@ def test_operators_put_again(monkeypatch):
     for step in (plan.evaluate_at_sources, lambda: plan.replay(tau), lambda: plan.build_expansions(tau)):
         with pytest.raises(ffmm.DeviceError, match="replaced"):
             step()
-    v = ffmm.DevicePlan(m, pts, ppl=20, bbox=BOX, cache=cache).matvec(tau).cpu().numpy()
+    new = ffmm.DevicePlan(m, pts, ppl=20, bbox=BOX, cache=cache)
+    v = new.matvec(tau).cpu().numpy()
     v_ref = O.FMM(cache.host_operators(), pts, 20, BOX[0], BOX[1]).matvec(tau)
     assert np.max(np.abs(v - v_ref)) < 1e-11 * np.max(np.abs(v_ref))
+    new.set_tol(1e-6)            # factors put before keep the other form's order
+    with pytest.raises(ffmm.DeviceError, match="replaced"):
+        new.build_expansions(tau)
