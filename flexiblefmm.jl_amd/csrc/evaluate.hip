@@ -15,7 +15,6 @@
 #include "ffmm_internal.h"
 
 #include <algorithm>
-#include <cstring>
 
 namespace ffmm {
 
@@ -274,86 +273,6 @@ __global__ void __launch_bounds__(EVT) k_eval32(EvalArgs a) {
       }
     }
   }
-}
-
-// Per leaf with points: points x near sources, their sum and maximum and the number of such
-// leaves, for eval_wide.  Two launches of some 5 us in a plan, read with its last synchronisation.
-constexpr int NW_B = 64, NW_SLOT = 60;   // blocks; first of three pinned slots, above the per-level ones
-static_assert(NW_SLOT >= 2 + 2 * (MAX_KEY_LEVELS + 2) && NW_SLOT + 3 <= NPINNED - 1, "free pinned slots");
-__device__ __forceinline__ void near_work_block(double &sum, double &top, double &cnt, double red[3][4]) {
-  for (int off = 32; off > 0; off >>= 1) {
-    sum += __shfl_xor(sum, off, 64);
-    top = fmax(top, __shfl_xor(top, off, 64));
-    cnt += __shfl_xor(cnt, off, 64);
-  }
-  const int w = threadIdx.x / 64, nw = blockDim.x / 64;
-  if (threadIdx.x % 64 == 0) {
-    red[0][w] = sum;
-    red[1][w] = top;
-    red[2][w] = cnt;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0)
-    for (int i = 1; i < nw; i++) {
-      sum += red[0][i];
-      top = fmax(top, red[1][i]);
-      cnt += red[2][i];
-    }
-}
-__global__ void __launch_bounds__(TB) k_near_work(const int32_t *__restrict__ leaves, int64_t n,
-                                                  const int32_t *__restrict__ col, int64_t nn,
-                                                  const int32_t *__restrict__ plo, const int32_t *__restrict__ phi,
-                                                  double *__restrict__ part) {
-  __shared__ double red[3][TB / 64];
-  double sum = 0.0, top = 0.0, cnt = 0.0;
-  for (int64_t q = (int64_t)blockIdx.x * TB + threadIdx.x; q < n; q += (int64_t)NW_B * TB) {
-    const int32_t i = leaves[q];
-    const double own = max(0, phi[i] - plo[i] + 1);
-    if (own == 0.0) continue;
-    double near = 0.0;
-    for (int k = 0; k < NCOLL; k++) {
-      const int32_t j = col[(int64_t)k * nn + i];
-      if (j >= 0) near += max(0, phi[j] - plo[j] + 1);
-    }
-    sum += own * near;
-    top = fmax(top, own * near);
-    cnt += 1.0;
-  }
-  near_work_block(sum, top, cnt, red);
-  if (threadIdx.x == 0) {
-    part[3 * blockIdx.x] = sum;
-    part[3 * blockIdx.x + 1] = top;
-    part[3 * blockIdx.x + 2] = cnt;
-  }
-}
-__global__ void __launch_bounds__(NW_B) k_near_total(const double *__restrict__ part, int64_t *__restrict__ host) {
-  __shared__ double red[3][4];
-  double sum = part[3 * threadIdx.x], top = part[3 * threadIdx.x + 1], cnt = part[3 * threadIdx.x + 2];
-  near_work_block(sum, top, cnt, red);
-  if (threadIdx.x == 0) {
-    host[0] = __double_as_longlong(sum);
-    host[1] = __double_as_longlong(top);
-    host[2] = (int64_t)cnt;
-  }
-}
-void near_work(Plan &plan) {
-  const int64_t n = plan.leaf_off[plan.L];
-  if (n >= EVAL_WIDE_LEAVES) return;
-  Context &ctx = *plan.ctx;
-  DBuf<double> part;
-  part.resize(3 * NW_B);
-  k_near_work<<<NW_B, TB, 0, ctx.stream>>>(plan.leaf_nodes.p, n, plan.col.p, plan.nnodes, plan.plo.p, plan.phi.p, part.p);
-  k_near_total<<<1, NW_B, 0, ctx.stream>>>(part.p, ctx.pinned_dev + NW_SLOT);
-  FFMM_LAUNCH_CHECK();
-}
-void near_work_read(Plan &plan) {
-  plan.near_leaves = 0;
-  plan.near_sum = plan.near_max = 0.0;
-  if (plan.leaf_off[plan.L] >= EVAL_WIDE_LEAVES) return;
-  const int64_t *v = plan.ctx->pinned + NW_SLOT;
-  std::memcpy(&plan.near_sum, v, sizeof(double));
-  std::memcpy(&plan.near_max, v + 1, sizeof(double));
-  plan.near_leaves = v[2];
 }
 
 static void launch_eval(Plan &plan, EvalArgs &a, int output, int64_t ntargets) {

@@ -138,7 +138,8 @@ void context_init(Context &c, int device, void *stream) {
   FFMM_BLAS(rocblas_create_handle(&c.blas));
   FFMM_BLAS(rocblas_set_stream(c.blas, c.stream));
   FFMM_BLAS(rocblas_set_pointer_mode(c.blas, rocblas_pointer_mode_host));
-  FFMM_HIP(hipHostMalloc((void **)&c.pinned, 64 * sizeof(int64_t), hipHostMallocMapped | hipHostMallocCoherent));
+  FFMM_HIP(hipHostMalloc((void **)&c.pinned, (NPINNED + 3 * NPINNED_WORK) * sizeof(int64_t),
+                         hipHostMallocMapped | hipHostMallocCoherent));
   FFMM_HIP(hipHostGetDevicePointer((void **)&c.pinned_dev, c.pinned, 0));
   // idle plan memory kept for reuse: up to half of the device's memory
   size_t fr = 0, tot = 0;
@@ -850,7 +851,6 @@ static void plan_finish(Plan &p) {
     p.khat.upload(kh.data(), p.L, ctx.stream);
   }
   node_leafslots(p);
-  near_work(p);
   {
     StageTimer tm(p, 1);
     build_lists(p);

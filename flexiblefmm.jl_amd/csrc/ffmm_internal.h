@@ -206,7 +206,7 @@ struct Context {
   bool own_stream = false;
   rocblas_handle blas = nullptr;
   std::unique_ptr<BlockCache> blocks = std::make_unique<BlockCache>();
-  int64_t *pinned = nullptr;   // small pinned readback area (64 entries), coherent
+  int64_t *pinned = nullptr;   // small pinned readback area (NPINNED slots, then NPINNED_WORK x 3), coherent
   int64_t *pinned_dev = nullptr;   // its device address: kernels store results there directly
   DBuf<char> tmp;               // scratch of the primitives
   void sync() { FFMM_HIP(hipStreamSynchronize(stream)); }
@@ -380,8 +380,8 @@ struct Plan {
   // node lists per level (concatenated): childless sourced nodes, real leaves
   std::vector<int64_t> s2m_off, leaf_off;   // L + 1 offsets
   DBuf<int32_t> s2m_nodes, leaf_nodes;
-  // plans of fewer than EVAL_WIDE_LEAVES leaves: those with points, and the sum and the
-  // largest of points x near sources over them
+  // where near_work_wanted: the leaves with points, and the sum and the largest of points x
+  // near sources over them
   int64_t near_leaves = 0;
   double near_sum = 0.0, near_max = 0.0;
   // the form and the largest rank of the cube operators that the buffers were made for
@@ -457,6 +457,7 @@ void compact_flags_u8_known(Context &ctx, const uint8_t *flag, int32_t *idx, int
 void compact_flags_u8_async(Context &ctx, const uint8_t *flag, int32_t *idx, int64_t n, int slot);
 void set_pinned(Context &ctx, int slot, int64_t v);
 constexpr int NPINNED = 64;
+constexpr int NPINNED_WORK = 64;   // behind them, three values for each block of k_leaf_slots
 
 // ---- tree (tree.hip) ----
 void bounds(Context &ctx, const double *xyz, int64_t n, double lo[3], double hi[3], int *all_finite);
@@ -630,20 +631,30 @@ __device__ __forceinline__ f32x2 unpack_bf16(uint32_t b) {
 //   Yukawa mixed     .055 / .111       .319 / .367     .050 / .136     .309 / .270    .303 / .464
 // Over 140 plans and 0.5 to 16 targets a leaf the rule loses 0.5 to 1.5% on average to the
 // better of the two, 1.3 times at most; the number of leaves alone lost up to 2.7 times.
+// Below `share` leaves no largest leaf is needed to know: four waves.
 constexpr int64_t EVAL_WIDE_LEAVES = 16384, EVAL_WIDE_LEAVES_YUKAWA = 6144;
-inline bool eval_wide(const Plan &plan, int64_t ntargets) {
-  constexpr double FIXED = 3200.0;
+inline int64_t eval_share(const Plan &plan) {
   const OpCache &o = *plan.ops;
-  const bool yukawa = o.kernel == FFMM_KERNEL_YUKAWA;
-  const double share = o.method == METHOD_CUBE                ? 3600.0
-                       : yukawa                               ? 450.0
-                       : o.kernel == FFMM_KERNEL_LAPLACE      ? 3200.0
-                       : plan.precision == FFMM_PREC_MIXED    ? 1400.0
-                                                              : 900.0;
+  if (o.method == METHOD_CUBE) return 3600;
+  if (o.kernel == FFMM_KERNEL_YUKAWA) return 450;
+  if (o.kernel == FFMM_KERNEL_LAPLACE) return 3200;
+  return plan.precision == FFMM_PREC_MIXED ? 1400 : 900;
+}
+inline int64_t eval_wide_leaves(const Plan &plan) {
+  return plan.ops->method != METHOD_CUBE && plan.ops->kernel == FFMM_KERNEL_YUKAWA ? EVAL_WIDE_LEAVES_YUKAWA
+                                                                                  : EVAL_WIDE_LEAVES;
+}
+// whether the near field's work is needed: the plan's leaves between the two bounds
+inline bool near_work_wanted(const Plan &plan) {
+  const int64_t n = plan.leaf_off[plan.L];
+  return n >= eval_share(plan) && n < eval_wide_leaves(plan);
+}
+inline bool eval_wide(const Plan &plan, int64_t ntargets) {
+  if (!near_work_wanted(plan)) return plan.leaf_off[plan.L] < eval_share(plan);
+  constexpr double FIXED = 3200.0;
   const double f = (double)ntargets / (double)plan.N;
   const double leaves = (double)std::min(plan.near_leaves, ntargets);
-  return plan.leaf_off[plan.L] < (yukawa ? EVAL_WIDE_LEAVES_YUKAWA : EVAL_WIDE_LEAVES) &&
-         leaves * FIXED + plan.near_sum * f < share * (plan.near_max * f + FIXED);
+  return leaves * FIXED + plan.near_sum * f < (double)eval_share(plan) * (plan.near_max * f + FIXED);
 }
 
 // sums of the replicas of each of ntp targets (thread t: target t % ntp) into the threads
@@ -742,8 +753,8 @@ size_t plan_bytes(const Plan &p);
 // ---- harmonic methods (harmonic.hip) ----
 void harmonic_s2m_level(Plan &plan, int l);
 void launch_eval_harmonic(Plan &plan, const EvalArgs &a, int output, bool wide);
-// the near field's work by leaf, queued; near_work_read after the stream's next synchronisation
-void near_work(Plan &plan);
+// the near field's work by leaf, from the blocks' shares that node_leafslots left in pinned
+// memory, after the stream's next synchronisation
 void near_work_read(Plan &plan);
 
 // ---- timing ----

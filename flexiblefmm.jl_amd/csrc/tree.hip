@@ -140,9 +140,54 @@ __global__ void k_fill_i32(int32_t *__restrict__ a, int64_t n, int32_t v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) a[i] = v;
 }
-__global__ void k_leaf_slots(const int32_t *__restrict__ leaf_nodes, int64_t nleaves, int32_t *__restrict__ slot) {
-  int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s < nleaves) slot[leaf_nodes[s]] = (int32_t)s;
+// With part, also each block's share of the near field's work for eval_wide: over the leaves with
+// points, the sum and the largest of points x near sources, and the number of these leaves.
+// The blocks' shares go to host memory with this launch, which a plan has anyway (two launches
+// of their own took 20 us of a 1.8 ms solve).
+__global__ void __launch_bounds__(TB) k_leaf_slots(const int32_t *__restrict__ leaves, int64_t n,
+                                                   int32_t *__restrict__ slot, const int32_t *__restrict__ col,
+                                                   int64_t nn, const int32_t *__restrict__ plo,
+                                                   const int32_t *__restrict__ phi, double *__restrict__ part) {
+  __shared__ double red[3][TB / 64];
+  const int64_t q = (int64_t)blockIdx.x * TB + threadIdx.x;
+  const int32_t i = q < n ? leaves[q] : -1;
+  if (i >= 0) slot[i] = (int32_t)q;
+  if (!part) return;
+  // all loads in flight at once: a colleague that is missing reads the leaf itself, uncounted
+  const int32_t self = max(i, 0);
+  int32_t j[NCOLL], own = phi[self] - plo[self] + 1, near = 0;
+#pragma unroll
+  for (int k = 0; k < NCOLL; k++) j[k] = col[(int64_t)k * nn + self];
+#pragma unroll
+  for (int k = 0; k < NCOLL; k++) {
+    const int32_t jj = j[k] >= 0 ? j[k] : self, cnt = phi[jj] - plo[jj] + 1;
+    near += j[k] >= 0 ? max(0, cnt) : 0;
+  }
+  const bool on = i >= 0 && own > 0;
+  const double work = on ? (double)own * (double)near : 0.0;
+  double cnt = on ? 1.0 : 0.0;
+  double sum = work, top = work;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    sum += __shfl_xor(sum, off, 64);
+    top = fmax(top, __shfl_xor(top, off, 64));
+    cnt += __shfl_xor(cnt, off, 64);
+  }
+  if (threadIdx.x % 64 == 0) {
+    red[0][threadIdx.x / 64] = sum;
+    red[1][threadIdx.x / 64] = top;
+    red[2][threadIdx.x / 64] = cnt;
+  }
+  __syncthreads();
+  if (threadIdx.x > 0) return;
+  for (int w = 1; w < TB / 64; w++) {
+    sum += red[0][w];
+    top = fmax(top, red[1][w]);
+    cnt += red[2][w];
+  }
+  part[3 * blockIdx.x] = sum;
+  part[3 * blockIdx.x + 1] = top;
+  part[3 * blockIdx.x + 2] = cnt;
 }
 
 struct DevLevel {
@@ -627,8 +672,24 @@ void node_leafslots(Plan &plan) {
   const int64_t nleaves = plan.leaf_off[plan.L];
   plan.node_leafslot.resize(plan.nnodes);
   k_fill_i32<<<nblocks(plan.nnodes, TB), TB, 0, s>>>(plan.node_leafslot.p, plan.nnodes, -1);
-  k_leaf_slots<<<nblocks(nleaves, TB), TB, 0, s>>>(plan.leaf_nodes.p, nleaves, plan.node_leafslot.p);
+  static_assert(EVAL_WIDE_LEAVES <= (int64_t)NPINNED_WORK * TB, "a share of the pinned memory per block");
+  double *part = near_work_wanted(plan) ? reinterpret_cast<double *>(plan.ctx->pinned_dev + NPINNED) : nullptr;
+  k_leaf_slots<<<nblocks(nleaves, TB), TB, 0, s>>>(plan.leaf_nodes.p, nleaves, plan.node_leafslot.p, plan.col.p,
+                                                   plan.nnodes, plan.plo.p, plan.phi.p, part);
   FFMM_LAUNCH_CHECK();
+}
+
+void near_work_read(Plan &plan) {
+  const int64_t nleaves = plan.leaf_off[plan.L];
+  plan.near_leaves = 0;
+  plan.near_sum = plan.near_max = 0.0;
+  if (!near_work_wanted(plan)) return;
+  const double *part = reinterpret_cast<const double *>(plan.ctx->pinned + NPINNED);
+  for (int64_t b = 0; b < nblocks(nleaves, TB); b++) {
+    plan.near_sum += part[3 * b];
+    plan.near_max = std::max(plan.near_max, part[3 * b + 1]);
+    plan.near_leaves += (int64_t)part[3 * b + 2];
+  }
 }
 
 }  // namespace ffmm

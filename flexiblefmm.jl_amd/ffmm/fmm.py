@@ -801,7 +801,8 @@ class DevicePlan:
 
     def near_work(self):
         """The sum and the largest of points × near sources over the leaves with points, and
-        the number of these (zeros for a plan of 16,384 leaves or more)."""
+        the number of these (zeros where the number of leaves alone decides how the
+        evaluation is launched)."""
         out = np.zeros(3)
         call("ffmm_plan_near_work", self._h, out.ctypes.data_as(ctypes.c_void_p))
         return out

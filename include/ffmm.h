@@ -320,8 +320,9 @@ int ffmm_plan_stage_times(ffmm_plan plan, double *ms, int n);
 int ffmm_plan_spectral_tiles(ffmm_plan plan, int64_t *staged, int64_t *cut, int n);
 /* The near field's work of the leaves with points, which the evaluation's launch is chosen by:
  * out[0] the sum and out[1] the largest of a leaf's points x near sources, out[2] the number
- * of such leaves; zeros for a plan of 16,384 leaves or more.  No reference counterpart: a
- * diagnostic. */
+ * of such leaves; zeros for a plan whose number of leaves decides by itself (below 3,600 or
+ * from 16,384 on, cube method; Laplace 3,200, Stokes 1,400 mixed and 900 FP64, Yukawa 450 and
+ * 6,144).  No reference counterpart: a diagnostic. */
 int ffmm_plan_near_work(ffmm_plan plan, double out[3]);
 
 /* ---- serving: continuous batching of solves on one device ----

@@ -104,16 +104,18 @@ def test_few_leaves_vs_one_wave(kernel, p, bound, precision, tol):
     assert np.linalg.norm(c - a[order]) < tol * np.linalg.norm(a[order])
 
 
-@pytest.mark.parametrize("n,ppl", [(1, 5), (90, 4), (2000, 3), (20_000, 3), (30_000, 40), (60_000, 2)])
-def test_near_work_vs_tree(n, ppl):
-    """The work that the evaluation's launch is chosen by against the downloaded tree: one
-    leaf, one block's and several blocks' leaves, empty ones; none for a plan of 16,384
-    leaves.  Whole numbers, so equal."""
+@pytest.mark.parametrize("n,ppl", [(1, 5), (90, 4), (600, 3), (2000, 3), (30_000, 40), (60_000, 2)])
+@pytest.mark.parametrize("kernel,lo,hi", [("cube", 3600, 16384), ("yukawa", 450, 6144)])
+def test_near_work_vs_tree(kernel, lo, hi, n, ppl):
+    """The work that the evaluation's launch is chosen by against the downloaded tree: several
+    blocks' leaves, empty ones; none where the number of leaves decides.  Whole numbers, so
+    equal."""
     import ffmm
     rng = np.random.default_rng(n)
     pts = rng.random((n, 3))
     pts[: n // 3] = 0.4 + 0.01 * rng.random((n // 3, 3))
-    m = ffmm.CubeKernelIndependent(ffmm.Laplace3D(), p=2)
+    m = (ffmm.CubeKernelIndependent(ffmm.Laplace3D(), p=2) if kernel == "cube"
+         else ffmm.SphericalHarmonics(ffmm.Yukawa3D(5.0), p=2))
     plan = ffmm.DevicePlan(m, pts, ppl=ppl, bbox=BOX)
     t = plan.download_tree()
     leaf = (t.leaf != 0) & (t.ghost == 0)
@@ -121,6 +123,6 @@ def test_near_work_vs_tree(n, ppl):
     cnt = np.maximum(t.phi - t.plo + 1, 0).astype(np.int64)
     col = t.colleagues[leaf]
     q = cnt[leaf] * np.where(col >= 0, cnt[np.maximum(col, 0)], 0).sum(1)
-    want = [q.sum(), q.max(), (cnt[leaf] > 0).sum()] if leaf.sum() < 16384 else [0, 0, 0]
-    print(f"[eval wide] near work n={n}: {leaf.sum()} leaves", flush=True)
+    print(f"[eval wide] near work {kernel} n={n}: {leaf.sum()} leaves", flush=True)
+    want = [q.sum(), q.max(), (cnt[leaf] > 0).sum()] if lo <= leaf.sum() < hi else [0, 0, 0]
     assert np.array_equal(plan.near_work(), np.array(want, dtype=np.float64))
