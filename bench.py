@@ -50,26 +50,27 @@ def interaction_counts(tree, nleaf_targets=None):
     return leaves, cnt[leaves], n[leaves]
 
 
-def gemm_shapes(plan, ops, mixed: bool):
-    """The dense products of one step of the cube method, in launch order: (name, m, n, k, type,
-    flop, library).  They size the step's work in its plain form; where the reflections of the
-    surfaces serve (even orders up to 10) the library runs them as eight blocks of an eighth of
-    the size, M2M in FP64.  Per step: UC2E as two FP64 factors over the childless sourced nodes of
-    levels 2 and below, M2M per level (FP32 in the mixed form, in calls of at most 10,240
-    columns) from level L-2 up to 2, L2L
-    per level (FP64) from level 3 down, DC2E as two FP64 factors over the leaves."""
+def blocks_serve(ops) -> bool:
+    """Whether the cube operators are applied as the reflections' 8 blocks (csrc/sym.hip), in
+    kernels of the library's own, rather than as dense BLAS products."""
+    return (ops.p in (2, 4, 6, 8, 10) and ops.pc % 2 == 0
+            and ops.P_up.rank == ops.nsmall and ops.P_down.rank == ops.nsmall)
+
+
+def gemm_shapes(plan, ops, mixed: bool, blocks: bool = False):
+    """The products of one step of the cube method, in launch order: (name, m, n, k, type, flop,
+    library: run by the BLAS library).  Per step: UC2E as two FP64 factors over the childless
+    sourced nodes of levels 2 and below, M2M per level from level L-2 up to 2, L2L per level
+    (FP64) from level 3 down, DC2E as two FP64 factors over the leaves.  Dense, M2M is FP32 in
+    the mixed form, in calls of at most 10,240 columns; as blocks, each product is 8 of an
+    eighth of its rows and columns (m and k are one block's), FP64 in both forms."""
     Ns, Nl, L = ops.nsmall, ops.nlarge, plan.nlevels
     nq_up, nq_dn = int(plan.level_s2m[2:].sum()), int(plan.level_leaves[2:].sum())
     ru, rd = ops.P_up.rank, ops.P_down.rank
-    # the labels of the p = 8 products name the kernels of an earlier form; they stay, so that
-    # records compare
-    fused = 241 <= ru <= 304
-    cols_up, cols_dn = 240 < Ns <= 304, 240 < rd <= 304
-    out = [("UC2E Uh" + (" (in k_s2m_uc2e)" if fused else ""), ru, nq_up, Nl, "f64"),
-           ("UC2E V" + (" (in k_gemm_cols)" if cols_up else ""), Ns, nq_up, ru, "f64")]
+    out = [("UC2E Uh", ru, nq_up, Nl, "f64"), ("UC2E V", Ns, nq_up, ru, "f64")]
     for l in range(L - 2, 1, -1):
         ng = int(plan.level_count[l + 1]) // 8
-        if mixed:   # the FP32 M2M runs in calls of at most 10,240 columns
+        if mixed and not blocks:
             for c0 in range(0, ng, 10240):
                 part = f" (columns {c0}-{min(ng, c0 + 10240) - 1})" if ng > 10240 else ""
                 out.append((f"M2M level {l}{part}", Ns, min(10240, ng - c0), 8 * Ns, "f32"))
@@ -77,15 +78,17 @@ def gemm_shapes(plan, ops, mixed: bool):
             out.append((f"M2M level {l}", Ns, ng, 8 * Ns, "f64"))
     for l in range(3, L):
         out.append((f"L2L level {l}", 8 * Ns, int(plan.level_count[l]) // 8, Ns, "f64"))
-    out += [("DC2E Uh" + (" (in k_gemm_cols)" if cols_dn else ""), rd, nq_dn, Ns, "f64"), ("DC2E V", Nl, nq_dn, rd, "f64")]
-    return [{"name": a, "m": m_, "n": n_, "k": k_, "type": t_, "flop": 2.0 * m_ * n_ * k_, "library": " (in " not in a}
+    out += [("DC2E Uh", rd, nq_dn, Ns, "f64"), ("DC2E V", Nl, nq_dn, rd, "f64")]
+    b = 8 if blocks else 1
+    return [{"name": a + (" (8 blocks)" if blocks else ""), "m": m_ // b, "n": n_, "k": k_ // b, "type": t_,
+             "flop": 2.0 * m_ * n_ * k_ / b, "library": not blocks}
             for a, m_, n_, k_, t_ in out if m_ > 0 and n_ > 0]
 
 
 def traffic_from_profile(kname: str, args):
-    """HBM bytes per launch of the dominant kernel from the committed two-pass
-    rocprofv3 --pmc profile (FETCH_SIZE, then WRITE_SIZE, each scaled by the copy
-    probe's reading), when the profile is of this kernel at this workload; else None."""
+    """HBM bytes per launch of the dominant kernel from the committed rocprofv3 --pmc profile
+    (FETCH_SIZE, then WRITE_SIZE, each scaled by the copy probe's reading), when the profile
+    is of this kernel at this workload; else None."""
     path = os.path.join(ROOT, "profiles", "hadamard_spectral_4M_mixed_traffic.json")
     if not os.path.exists(path) or args.n != 4_000_000 or args.ppl != 64:
         return None
@@ -646,7 +649,8 @@ def main():
 
     tree_stats = {"levels": plan.nlevels, "nodes": plan.nnodes, "far_pairs": int(plan.level_pairs.sum()),
                   "leaves": int(plan.level_leaves.sum()),
-                  "gemms": gemm_shapes(plan, cache.host_operators(), args.precision == "mixed")}
+                  "gemms": gemm_shapes(plan, cache.host_operators(), args.precision == "mixed",
+                                       blocks_serve(cache.host_operators()))}
     serving = None
     if args.serve_requests > 0:
         del plan                 # the measured plan's device memory goes back before the stream

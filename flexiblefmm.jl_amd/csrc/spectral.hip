@@ -263,14 +263,18 @@ __global__ void __launch_bounds__(64 * SpBoxes<T>::NB) k_spec_inverse(const type
 //
 // FP64: v_mfma_f64_16x16x4, 4 waves each over a quarter of the colleagues, two workgroups per
 // CU.  Measured: 300k sources 9.0 -> 4.5 ms (the products on the vector ALUs before, bound by
-// LDS); the matrix cores are busy half the time.  Mixed: each FP32 value as three bfloat16 pieces (8 significant bits
-// each: the whole FP32 mantissa), the products of pieces down to 2^-24 on
-// v_mfma_f32_16x16x32_bf16: hi hi in one FP32 accumulator; hi mid, mid hi, hi lo, lo hi and
-// mid mid in another.  Six bfloat16 products cost 96 cycles per 64 x 16 block of 32 K where
-// v_mfma_f32_16x16x4 takes 256, and a K of 32 per instruction rounds the sums less often:
-// against 64 bits the potential's error fell from 2.5e-7 to 1.1e-7 at 1M mixture sources.
-// Measured: 4M sources 17.1 -> 8.0 ms; bound by LDS (46% of its cycles), vector ALU (33%) and
-// matrix cores (26%) in turn, the fetches running at 1.5 TB/s.
+// LDS); the matrix cores are busy half the time.
+// Mixed: each FP32 value as three bfloat16 pieces (8 significant bits each: the whole FP32
+// mantissa), the products of pieces down to 2^-24 on v_mfma_f32_16x16x32_bf16 in three FP32
+// accumulators: hi hi; mid hi and hi mid; lo hi, mid mid and hi lo.  Six bfloat16 products cost
+// 96 cycles per 64 x 16 block of 32 K where v_mfma_f32_16x16x4 takes 256, and a K of 32 per
+// instruction rounds the sums less often: against 64 bits the potential's error fell from
+// 2.5e-7 to 1.1e-7 at 1M mixture sources.  The pieces of values below some 2^-110 leave
+// bfloat16's range: with charges of 2^-112 (2e-34) the error is as above, of 2^-116 2.5e-7,
+// of 2^-120 3.6e-6 (FP32 operands 1.4e-7), of 2^-126 2.5e-4 (1.9e-6).
+// Measured: 4M sources 17.1 -> 8.0 ms; bound by LDS (active 67% of the cycles, half of that
+// counted as bank conflicts), then vector ALU (51%) and matrix cores (33%); 1.78 GB fetched
+// and 0.46 GB written a level, 2.8 TB/s.
 // ---------------------------------------------------------------------------
 constexpr int HM_TILE = 16;          // sibling groups per tile: the matrix instructions' columns
 typedef double f64x4 __attribute__((ext_vector_type(4)));

@@ -106,3 +106,24 @@ def test_bench_gemm_record_splits_the_wide_mixed_m2m():
                      "L2L level 3", "L2L level 4", "L2L level 5", "DC2E Uh", "DC2E V"]
     # narrower levels are one call, named as before
     assert [g["name"] for g in mixed if g["name"].startswith("M2M level 4")] == ["M2M level 4"]
+
+
+def test_bench_gemm_record_of_blocks():
+    """The same record where the reflections' blocks serve: one FP64 entry per product and
+    level, each 8 products of an eighth of the rows and columns, none run by the library."""
+    import types
+    import bench
+    Ns, Nl = 296, 1352
+    ops = types.SimpleNamespace(p=8, pc=16, nsmall=Ns, nlarge=Nl, P_up=types.SimpleNamespace(rank=296),
+                                P_down=types.SimpleNamespace(rank=296))
+    assert bench.blocks_serve(ops)
+    assert not bench.blocks_serve(types.SimpleNamespace(**{**vars(ops), "pc": 15}))
+    assert not bench.blocks_serve(types.SimpleNamespace(**{**vars(ops), "P_up": types.SimpleNamespace(rank=292)}))
+    counts = np.array([1, 8, 64, 512, 8 * 25_000, 800])
+    plan = types.SimpleNamespace(nlevels=len(counts), level_count=counts, level_s2m=np.full(len(counts), 1000),
+                                 level_leaves=np.full(len(counts), 900))
+    dense, blocks = bench.gemm_shapes(plan, ops, False), bench.gemm_shapes(plan, ops, True, True)
+    assert [g["name"] for g in blocks] == [g["name"] + " (8 blocks)" for g in dense]
+    for d, b in zip(dense, blocks):
+        assert (8 * b["m"], b["n"], 8 * b["k"]) == (d["m"], d["n"], d["k"]) and b["type"] == "f64"
+        assert b["flop"] == d["flop"] / 8 == 8 * 2.0 * b["m"] * b["n"] * b["k"] and not b["library"]
