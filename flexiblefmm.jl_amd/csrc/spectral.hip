@@ -865,6 +865,9 @@ void spectral_prepare(Plan &plan) {
   v.L = L;
   for (int l = 2; l < L; l++) {
     const int64_t ng = plan.nl[l] / NCHILD;
+    // k_group_cols keeps a box's place in the level in 23 bits (such a level's spectra alone
+    // take 226 GB in the mixed form)
+    if (plan.nl[l] > (1 << 23)) fail(FFMM_ERR_ARGUMENT, "too many boxes on one level for the spectral M2L");
     v.lo[l] = plan.lo[l];
     v.goff[l + 1] = v.goff[l] + ng;
     v.toff[l + 1] = plan.spec_tile0[l + 1] = v.toff[l] + (ng + HM_TILE - 1) / HM_TILE;

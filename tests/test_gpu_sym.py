@@ -140,12 +140,27 @@ def test_given_operators_are_applied(p, given, precision):
         assert np.max(np.abs(u - u_ref)) < 1e-11 * np.max(np.abs(u_ref))
 
 
+def _put_again(cache, monkeypatch):
+    """Put the cache's host operators again into its device copy."""
+    from ffmm import fmm as F
+    h, call = cache.device(0), F.call
+
+    def put(name, *args):
+        if name == "ffmm_opcache_create":
+            args[-1]._obj.value = h.value
+        else:
+            call(name, *args)
+    cache._device.clear()
+    monkeypatch.setattr(F, "call", put)
+    cache.device(0)
+    monkeypatch.setattr(F, "call", call)
+
+
 def test_operators_put_again(monkeypatch):
     """Operators put again into a cache that a plan was made with: of the same form, the plan
     serves them; of the other form (here a scaled inverse, applied as given), the plan's
     passes, its evaluation and its captured replay are refused, and a new plan is right."""
     import ffmm
-    from ffmm import fmm as F
     rng = np.random.default_rng(4)
     pts, tau = rng.random((1500, 3)), rng.standard_normal(1500)
     m = ffmm.CubeKernelIndependent(ffmm.Laplace3D(), p=4)
@@ -153,23 +168,10 @@ def test_operators_put_again(monkeypatch):
     plan = ffmm.DevicePlan(m, pts, ppl=20, bbox=BOX, cache=cache).capture()
     u = plan.matvec(tau).cpu().numpy()
     cache.class_factors(0, 1e-6)
-    h, call = cache.device(0), F.call
-
-    def put_again(name, *args):
-        if name == "ffmm_opcache_create":
-            args[-1]._obj.value = h.value
-        else:
-            call(name, *args)
-
-    def again():
-        cache._device.clear()
-        monkeypatch.setattr(F, "call", put_again)
-        cache.device(0)
-        monkeypatch.setattr(F, "call", call)
-    again()
+    _put_again(cache, monkeypatch)
     assert np.array_equal(plan.matvec(tau).cpu().numpy(), u)
     cache.host_operators().P_up.invS *= 2.0
-    again()
+    _put_again(cache, monkeypatch)
     for step in (plan.evaluate_at_sources, lambda: plan.replay(tau), lambda: plan.build_expansions(tau)):
         with pytest.raises(ffmm.DeviceError, match="replaced"):
             step()
@@ -180,3 +182,24 @@ def test_operators_put_again(monkeypatch):
     new.set_tol(1e-6)            # factors put before keep the other form's order
     with pytest.raises(ffmm.DeviceError, match="replaced"):
         new.build_expansions(tau)
+
+
+@pytest.mark.parametrize("p,pc,d,width", [(2, 4, 0.1, 1.0), (4, 8, 0.3, 0.7361), (6, 12, 0.1, 1e-5), (8, 16, 0.1, 1.0),
+                                          (8, 16, 0.01, 3.3e4), (8, 24, 0.6, 1.0), (8, 8, 0.1, 0.3), (10, 20, 0.1, 1.0),
+                                          (10, 20, 0.05, 17.0)])
+def test_default_operators_take_the_blocks(p, pc, d, width, monkeypatch):
+    """The library's own operators pass the checks of the blocks at every order, surface and
+    width: a scaled inverse put afterwards is of the other form, which a plan of the first
+    refuses."""
+    import ffmm
+    print(f"[sym] form of p={p} pc={pc} d={d} width={width}", flush=True)
+    rng = np.random.default_rng(p)
+    pts = width * rng.random((100, 3))
+    m = ffmm.CubeKernelIndependent(ffmm.Laplace3D(), p=p, pc=pc, d=d)
+    cache = ffmm.OperatorCache(m)
+    plan = ffmm.DevicePlan(m, pts, ppl=10, bbox=(np.zeros(3), width), cache=cache)
+    plan.matvec(rng.standard_normal(100))
+    cache.host_operators().P_up.invS *= 2.0
+    _put_again(cache, monkeypatch)
+    with pytest.raises(ffmm.DeviceError, match="replaced"):
+        plan.evaluate_at_sources()
