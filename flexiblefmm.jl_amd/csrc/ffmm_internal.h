@@ -619,8 +619,8 @@ __device__ __forceinline__ f32x2 unpack_bf16(uint32_t b) {
 // leaves the card's 1,024 SIMDs idle where there are few leaves, and lets the largest leaves end
 // last; four waves cost their barriers and the sum of their parts, which small leaves do not
 // pay back.  So the largest leaf's share of the work decides: four waves where it is more than
-// 1 / share, a leaf's work being its targets x near sources (near_work: those of the sources,
-// in proportion for other targets) and 3,200 such pairs for what does not depend on them.
+// 1 / share, a leaf's work being its targets x near sources (k_leaf_slots counts them for
+// the sources; other targets in proportion) and 3,200 such pairs for what does not depend on them.
 // Measured at the sources, one wave / four (ms; leaves, points a leaf; p = 8, Yukawa 10):
 //                  uniform, 4,096    uniform, 4,096    density ~ x^-1/3 an axis
 //                  leaves of 6       of 32             6,014 of 2.4    5,937 of 15    10,424 of 15

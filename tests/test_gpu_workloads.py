@@ -105,7 +105,7 @@ def test_mixture_mixed_spectral_targets(mixture):
     assert max(e) <= 1e-6
 
 
-def test_mixture_400k_mixed_spectral_both_hadamard_kernels():
+def test_mixture_400k_mixed_spectral_whole_and_cut_tiles():
     """400,000 Gaussian-mixture sources, mixed precision, spectral M2L. At this size a few
     tiles of 16 sibling groups name more than 192 distinct colleague boxes, so the
     Hadamard products run on tiles staged whole and on tiles cut into subtiles; the
